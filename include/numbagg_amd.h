@@ -280,6 +280,15 @@ int nbg_nanargmax(int dtype, const void* x, void* out, int64_t rows, int64_t n,
                   int64_t ld, void* ws, size_t ws_bytes, void* stream); /* funcs.py:160-178 */
 int nbg_nanargmin(int dtype, const void* x, void* out, int64_t rows, int64_t n,
                   int64_t ld, void* ws, size_t ws_bytes, void* stream); /* funcs.py:181-197 */
+/* The same reductions (name: the entry point above, "nbg_nanvar") over an axis
+ * that is not the innermost: element i of output (a, c) is x[a * ld_outer +
+ * i * ld_row + c], a < outer, i < n, c < cols; out is (outer, cols). ddof is
+ * read by nanvar and nanstd only. */
+size_t nbg_reduce_cols_workspace_bytes(int64_t outer, int64_t n, int64_t cols, int dtype);
+int nbg_reduce_cols(const char* name, int dtype, const void* x, void* out,
+                    int64_t outer, int64_t n, int64_t cols, int64_t ld_outer,
+                    int64_t ld_row, int64_t ddof, void* ws, size_t ws_bytes,
+                    void* stream);
 
 /* ---- label factorisation (the caller-side step before the grouped
  *      reductions: numbagg/decorators.py:570-573 requires factorised labels,

@@ -3,9 +3,11 @@
 // numbagg/decorators.py:188-272) and nanmax, nanmin, nanargmax, nanargmin
 // (ndreduce, numbagg/funcs.py:160-228, numbagg/decorators.py:904-1028).
 //
-// The host moves the reduced axes last and flattens them, so every kernel sees
+// The host moves the reduced axes last and flattens them, so a kernel sees
 // a row-major (rows, n) view with a unit-stride core axis and reduces each
-// row to one output.
+// row to one output; where the innermost axis is kept, it passes the
+// (outer, n, cols) view as it lies and the column kernel reduces it in place
+// (below), without a transposed copy.
 //
 // Design: one wavefront reduces one (row, chunk) item. Rows are split into
 // chunks so that a launch holds enough wavefronts to fill the device; each
@@ -23,6 +25,7 @@
 // passes over the data, numbagg/funcs.py:108-127); extremes as orderable
 // 64-bit keys with the index of the first (arg*: the reference replaces on a
 // strict `>` / `<`) or last (min/max: it replaces on `>=` / `<=`) occurrence.
+#include <cstring>
 #include <type_traits>
 
 #include "common.hpp"
@@ -76,6 +79,12 @@ __device__ __forceinline__ unsigned long long ext_key(T v, bool minimum) {
   const unsigned long long b = bits_of((double)v + 0.0);
   const unsigned long long k = (b & 0x8000000000000000ull) ? ~b : (b | 0x8000000000000000ull);
   return minimum ? ~k : k;
+}
+
+// 1/v for v >= 1: the hardware estimate refined by one Newton step.
+__device__ __forceinline__ double recip_refined(double v) {
+  const double r = __builtin_amdgcn_rcp(v);
+  return fma(r, fma(-v, r, 1.0), r);
 }
 
 // (count, mean, M2) and Chan's merge of another such triple.
@@ -184,6 +193,43 @@ struct Lane {
       m2b += !is_nan(v[j]) ? d * d : 0.0;
     }
     ch.merge((double)nb, mb, m2b);
+  }
+
+  // The same without float64 divisions: the batch mean from a refined
+  // reciprocal corrected by its remainder (so equal values have exactly their
+  // value as mean, and no variance), the merge's weight from a refined
+  // reciprocal (about 1 ULP).
+  template <int B>
+  __device__ __forceinline__ void fold_batch_rcp(const T (&v)[B]) {
+    double sb = 0.0;
+    int nb = 0;
+#pragma unroll
+    for (int j = 0; j < B; ++j) {
+      const bool valid = !is_nan(v[j]);
+      sb += valid ? (double)v[j] : 0.0;
+      nb += valid ? 1 : 0;
+    }
+    const double dn = (double)nb;
+    const double r = recip_refined(nb > 0 ? dn : 1.0);
+    const double q = sb * r;
+    const double mb = fma(fma(-dn, q, sb), r, q);
+    double m2b = 0.0;
+#pragma unroll
+    for (int j = 0; j < B; ++j) {
+      const double d = !is_nan(v[j]) ? (double)v[j] - mb : 0.0;
+      m2b = fma(d, d, m2b);
+    }
+    if (nb == 0) return;
+    if (ch.n == 0.0) {
+      ch = Chan{dn, mb, m2b};
+      return;
+    }
+    const double tot = ch.n + dn;
+    const double d = mb - ch.mean;
+    const double f = dn * recip_refined(tot);
+    ch.mean += d * f;
+    ch.m2 += m2b + d * d * ch.n * f;
+    ch.n = tot;
   }
 
   // c0: the chunk's first position (small_ext indices are relative to it).
@@ -341,10 +387,10 @@ __global__ __launch_bounds__(kRedThreads) void reduce_kernel(const T* __restrict
   if (lane == 0) parts[item] = p;
 }
 
-// The output of one row from its merged partial.
+// The output of one row from its merged partial; the row's element i is
+// x[i * step].
 template <typename T, typename TO, int KIND>
-__device__ __forceinline__ TO part_value(const RPart& p, int64_t row, int64_t ddof, const T* __restrict__ x,
-                                         int64_t ld) {
+__device__ __forceinline__ TO part_value(const RPart& p, int64_t ddof, const T* __restrict__ x, int64_t step) {
   TO r;
   if constexpr (KIND == kRSum) {
     if constexpr (!std::is_floating_point<T>::value) {
@@ -377,7 +423,7 @@ __device__ __forceinline__ TO part_value(const RPart& p, int64_t row, int64_t dd
     // the value at the extreme's index, through float64 as the reference's
     // float64 running extreme returns it (64-bit integers round there)
     if (p.w0 == 0ull) r = (TO)canonical_nan<double>();
-    else r = (TO)(double)x[row * ld + (int64_t)p.w1];
+    else r = (TO)(double)x[(int64_t)p.w1 * step];
   }
   return r;
 }
@@ -391,7 +437,7 @@ __global__ void reduce_finalize_kernel(const RPart* __restrict__ parts, int64_t 
   if (row >= rows) return;
   RPart p = parts[row * chunks_per_row];
   for (int64_t c = 1; c < chunks_per_row; ++c) merge_part<T, KIND>(p, parts[row * chunks_per_row + c]);
-  out[row] = part_value<T, TO, KIND>(p, row, ddof, x, ld);
+  out[row] = part_value<T, TO, KIND>(p, ddof, x + row * ld, 1);
 }
 
 // The same for rows of many chunks, a workgroup per row: each thread merges a
@@ -433,7 +479,154 @@ __global__ __launch_bounds__(kRedFinishThreads) void reduce_finalize_wide_kernel
       }
     }
   }
-  if (t == 0) out[row] = part_value<T, TO, KIND>(sp[0], row, ddof, x, ld);
+  if (t == 0) out[row] = part_value<T, TO, KIND>(sp[0], ddof, x + row * ld, 1);
+}
+
+// ---- reductions over an axis that is not the innermost -----------------------
+// x[a * ld_a + i * ld_r + c], a < outer, i < n, c < cols: every (a, c) reduces
+// its n elements. A workgroup takes `cl` column lanes (V neighbouring columns
+// each, one vector load per row) by 256 / cl row lanes of one (a, split): the
+// row lanes of few-column arrays read consecutive rows, so a wave's loads stay
+// contiguous for any column count. Each lane keeps U rows of loads in flight
+// and a private state per column, the row lanes merge pairwise in LDS in a
+// fixed order, and the splits' partials are merged in split order by the
+// finalize kernel (deterministic, no atomics).
+//
+// Bound by HBM: one streaming read of x. 16-byte accesses need element
+// alignment only, so any column offset and row stride takes the vector path.
+template <typename T, int V>
+struct alignas(alignof(T)) ColVec {
+  T v[V];
+};
+
+constexpr int kColUnroll = 8;
+
+template <typename T, int KIND, int V>
+__global__ __launch_bounds__(kRedThreads) void reduce_cols_kernel(const T* __restrict__ x, int64_t n, int64_t cols,
+                                                                  int64_t ld_a, int64_t ld_r, int cl,
+                                                                  int64_t col_tiles, int64_t splits, int64_t chunk,
+                                                                  int64_t total, RPart* __restrict__ parts) {
+  constexpr int U = kColUnroll;
+  __shared__ RPart sp[kRedThreads * V];
+  const int tid = threadIdx.x;
+  const int RL = kRedThreads / cl;
+  const int lc = tid % cl, rl = tid / cl;
+  const int64_t tile = blockIdx.x % col_tiles;
+  const int64_t rest = blockIdx.x / col_tiles;
+  const int64_t split = rest % splits, a = rest / splits;
+  const int64_t c = (tile * cl + lc) * V;
+  const int64_t i0 = split * chunk;
+  const int64_t i1 = i0 + chunk < n ? i0 + chunk : n;
+  const bool act = rl < RL && c < cols;
+  const int nv = act ? (int)(cols - c < V ? cols - c : V) : 0;
+  Lane<T, KIND> st[V];
+  auto fold_one = [&](int k, T v, int64_t i) {
+    if constexpr (is_var_kind(KIND)) {
+      const T b[1] = {v};
+      st[k].template fold_batch_rcp<1>(b);
+    } else if constexpr (small_ext<T, KIND>()) {
+      st[k].fold32(v, (uint32_t)(i - i0));
+    } else {
+      st[k].fold(v, i);
+    }
+  };
+  if (nv == V) {
+    using CV = ColVec<T, V>;
+    const T* p = x + a * ld_a + c;
+    int64_t i = i0 + rl;
+    for (; i + (U - 1) * RL < i1; i += U * RL) {
+      CV vv[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) vv[u] = load_stream(reinterpret_cast<const CV*>(p + (i + u * RL) * ld_r));
+#pragma unroll
+      for (int k = 0; k < V; ++k) {
+        if constexpr (is_var_kind(KIND)) {
+          T b[U];
+#pragma unroll
+          for (int u = 0; u < U; ++u) b[u] = vv[u].v[k];
+          st[k].template fold_batch_rcp<U>(b);
+        } else {
+#pragma unroll
+          for (int u = 0; u < U; ++u) fold_one(k, vv[u].v[k], i + u * RL);
+        }
+      }
+    }
+    for (; i < i1; i += RL) {
+      const CV q = load_stream(reinterpret_cast<const CV*>(p + i * ld_r));
+#pragma unroll
+      for (int k = 0; k < V; ++k) fold_one(k, q.v[k], i);
+    }
+  } else if (nv > 0) {  // the last columns, short of a vector
+    const T* p = x + a * ld_a + c;
+    for (int64_t i = i0 + rl; i < i1; i += RL)
+#pragma unroll
+      for (int k = 0; k < V; ++k)
+        if (k < nv) fold_one(k, p[i * ld_r + k], i);
+  }
+  RPart q[V];
+#pragma unroll
+  for (int k = 0; k < V; ++k) q[k] = st[k].to_part(i0);
+  if (RL > 1) {  // uniform
+#pragma unroll
+    for (int k = 0; k < V; ++k) sp[k * kRedThreads + tid] = q[k];
+    for (int s = 1; s < RL; s <<= 1) {
+      __syncthreads();
+      if (act && (rl & (2 * s - 1)) == 0 && rl + s < RL) {
+#pragma unroll
+        for (int k = 0; k < V; ++k) {
+          merge_part<T, KIND>(q[k], sp[k * kRedThreads + tid + s * cl]);
+          sp[k * kRedThreads + tid] = q[k];
+        }
+      }
+    }
+  }
+  if (act && rl == 0) {
+#pragma unroll
+    for (int k = 0; k < V; ++k)
+      if (k < nv) parts[split * total + a * cols + c + k] = q[k];
+  }
+}
+
+template <typename T, typename TO, int KIND>
+__global__ void reduce_cols_finalize_kernel(const RPart* __restrict__ parts, int64_t total, int64_t splits,
+                                            int64_t cols, int64_t ld_a, int64_t ld_r, int64_t ddof,
+                                            const T* __restrict__ x, TO* __restrict__ out) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= total) return;
+  RPart p = parts[q];
+  for (int64_t s = 1; s < splits; ++s) merge_part<T, KIND>(p, parts[s * total + q]);
+  const int64_t a = q / cols;
+  out[q] = part_value<T, TO, KIND>(p, ddof, x + a * ld_a + (q - a * cols), ld_r);
+}
+
+// The launch's shape: column lanes, tiles and row splits.
+struct ColShape {
+  int v, cl;
+  int64_t tiles, splits, chunk;
+};
+
+// Vectors of 16 bytes where they fill at least half a wave; columns split
+// evenly over the tiles. Row splits: about 8 workgroups per CU (2048: every
+// SIMD then holds 8 waves), each split at least two unrolled steps of every
+// row lane. (3653, 65160) float32 nanvar takes 255 tiles by 8 splits.
+inline ColShape col_shape(int64_t outer, int64_t n, int64_t cols, int elem) {
+  ColShape c{};
+  const int vmax = 16 / elem;
+  c.v = cols >= 32 * vmax ? vmax : 1;
+  const int64_t units = (cols + c.v - 1) / c.v;
+  c.tiles = (units + kWave - 1) / kWave;
+  c.cl = (int)((units + c.tiles - 1) / c.tiles);
+  const int64_t step = (int64_t)(kRedThreads / c.cl) * kColUnroll;
+  const int64_t base = outer * c.tiles;
+  int64_t splits = base > 0 ? (2048 + base - 1) / base : 1;
+  const int64_t most = n / (2 * step);
+  if (splits > most) splits = most;
+  if (splits < 1) splits = 1;
+  c.chunk = (n + splits - 1) / splits;
+  c.chunk = (c.chunk + step - 1) / step * step;
+  if (c.chunk < step) c.chunk = step;
+  c.splits = n > 0 ? (n + c.chunk - 1) / c.chunk : 1;
+  return c;
 }
 
 // Chunks per row: about 8 wavefronts per SIMD over the device, chunks of
@@ -507,24 +700,67 @@ int reduce_impl(const T* x, TO* out, int64_t rows, int64_t n, int64_t ld, int64_
   return check_hip(hipGetLastError(), "reduce_finalize_kernel launch");
 }
 
+template <typename T, typename TO, int KIND>
+int reduce_cols_impl(const T* x, TO* out, int64_t outer, int64_t n, int64_t cols, int64_t ld_a, int64_t ld_r,
+                     int64_t ddof, void* ws, size_t ws_bytes, hipStream_t s) {
+  constexpr int VEC = 16 / (int)sizeof(T);
+  const ColShape c = col_shape(outer, n, cols, (int)sizeof(T));
+  const int64_t total = outer * cols;
+  const size_t need = (size_t)(total * c.splits) * sizeof(RPart);
+  if (ws == nullptr || ws_bytes < need)
+    return set_error(NBG_ERR_INVALID, "reduce: workspace too small (%zu < %zu)", ws_bytes, need);
+  const int64_t blocks = outer * c.tiles * c.splits;
+  const int64_t fblocks = (total + 255) / 256;
+  // positions relative to a split are kept in 32 bits (float32 extremes)
+  if (blocks > 0x7fffffffLL || fblocks > 0x7fffffffLL || c.chunk > 0x7fffffffLL)
+    return set_error(NBG_ERR_INVALID, "reduce: too many rows");
+  RPart* parts = static_cast<RPart*>(ws);
+  if (c.v == VEC)
+    hipLaunchKernelGGL((reduce_cols_kernel<T, KIND, VEC>), dim3((unsigned)blocks), dim3(kRedThreads), 0, s, x, n,
+                       cols, ld_a, ld_r, c.cl, c.tiles, c.splits, c.chunk, total, parts);
+  else
+    hipLaunchKernelGGL((reduce_cols_kernel<T, KIND, 1>), dim3((unsigned)blocks), dim3(kRedThreads), 0, s, x, n, cols,
+                       ld_a, ld_r, c.cl, c.tiles, c.splits, c.chunk, total, parts);
+  if (int rc = check_hip(hipGetLastError(), "reduce_cols_kernel launch")) return rc;
+  hipLaunchKernelGGL((reduce_cols_finalize_kernel<T, TO, KIND>), dim3((unsigned)fblocks), dim3(256), 0, s, parts,
+                     total, c.splits, cols, ld_a, ld_r, ddof, x, out);
+  return check_hip(hipGetLastError(), "reduce_cols_finalize_kernel launch");
+}
+
+// The (rows, n) view of a reduction (cols == 0: element i of row r is
+// x[r * ld + i]), or its (outer, n, cols) view (element i of (a, c) is
+// x[a * ld_a + i * ld + c]).
+struct RView {
+  int64_t rows, n, ld, cols, ld_a;
+};
+
 // Output dtype per kind: sum -> input; mean/var/std -> input (floats only);
 // count, argmax, argmin -> int64; allnan/anynan -> uint8 (bool); max/min ->
 // input for floats, int64 for integers.
 template <int KIND>
-int reduce_entry(const char* name, int dtype, const void* x, void* out, int64_t rows, int64_t n, int64_t ld,
-                 int64_t ddof, void* ws, size_t ws_bytes, void* stream) {
+int reduce_view(const char* name, int dtype, const void* x, void* out, const RView& w, int64_t ddof, void* ws,
+                size_t ws_bytes, void* stream) {
+  const int64_t rows = w.rows, n = w.n, ld = w.ld;
   if (int rc = injected_error(name)) return rc;
   if (rows < 0 || n < 0) return set_error(NBG_ERR_INVALID, "%s: negative shape", name);
   if (rows == 0) return NBG_OK;
   if ((x == nullptr && n > 0) || out == nullptr) return set_error(NBG_ERR_INVALID, "%s: null pointer", name);
-  if (rows > 1 && ld < n) return set_error(NBG_ERR_INVALID, "%s: row stride < n", name);
+  if (w.cols == 0 && rows > 1 && ld < n) return set_error(NBG_ERR_INVALID, "%s: row stride < n", name);
+  if (w.cols > 0 && ((n > 1 && ld < w.cols) || (rows > 1 && w.ld_a < 0)))
+    return set_error(NBG_ERR_INVALID, "%s: row stride < cols", name);
   if (n == 0 && (KIND == kRArgMax || KIND == kRArgMin || KIND == kRMax || KIND == kRMin))
     return set_error(NBG_ERR_INVALID, "%s: zero-size reduction", name);
   constexpr bool FLOAT_ONLY = KIND == kRMean || is_var_kind(KIND);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const bool flt = dtype == NBG_F32 || dtype == NBG_F64;
   if (FLOAT_ONLY && !flt) return set_error(NBG_ERR_INVALID, "%s: float32 or float64 input required", name);
-#define NBG_R(T, TO) return reduce_impl<T, TO, KIND>((const T*)x, (TO*)out, rows, n, ld, ddof, ws, ws_bytes, s)
+#define NBG_R(T, TO)                                                                                          \
+  do {                                                                                                        \
+    if (w.cols > 0)                                                                                           \
+      return reduce_cols_impl<T, TO, KIND>((const T*)x, (TO*)out, rows, n, w.cols, w.ld_a, ld, ddof, ws,      \
+                                           ws_bytes, s);                                                      \
+    return reduce_impl<T, TO, KIND>((const T*)x, (TO*)out, rows, n, ld, ddof, ws, ws_bytes, s);               \
+  } while (0)
   if constexpr (KIND == kRCount || KIND == kRArgMax || KIND == kRArgMin) {
     switch (dtype) {
       case NBG_F32: NBG_R(float, int64_t);
@@ -563,10 +799,46 @@ int reduce_entry(const char* name, int dtype, const void* x, void* out, int64_t 
   return set_error(NBG_ERR_INVALID, "%s: unsupported dtype code %d", name, dtype);
 }
 
+template <int KIND>
+int reduce_entry(const char* name, int dtype, const void* x, void* out, int64_t rows, int64_t n, int64_t ld,
+                 int64_t ddof, void* ws, size_t ws_bytes, void* stream) {
+  return reduce_view<KIND>(name, dtype, x, out, RView{rows, n, ld, 0, 0}, ddof, ws, ws_bytes, stream);
+}
+
 }  // namespace
 }  // namespace nbg
 
 extern "C" {
+
+size_t nbg_reduce_cols_workspace_bytes(int64_t outer, int64_t n, int64_t cols, int dtype) {
+  if (outer <= 0 || cols <= 0 || n < 0) return 0;
+  const int elem = (dtype == NBG_F64 || dtype == NBG_I64) ? 8 : 4;
+  return (size_t)(outer * cols * nbg::col_shape(outer, n, cols, elem).splits) * sizeof(nbg::RPart);
+}
+
+int nbg_reduce_cols(const char* name, int dtype, const void* x, void* out, int64_t outer, int64_t n, int64_t cols,
+                    int64_t ld_outer, int64_t ld_row, int64_t ddof, void* ws, size_t ws_bytes, void* stream) {
+  using namespace nbg;
+  if (name == nullptr) return set_error(NBG_ERR_INVALID, "nbg_reduce_cols: null name");
+  if (cols < 0) return set_error(NBG_ERR_INVALID, "%s: negative shape", name);
+  if (cols == 0) return NBG_OK;
+  const RView w{outer, n, ld_row, cols, ld_outer};
+#define NBG_COLS(NAME, KIND) \
+  if (strcmp(name, NAME) == 0) return reduce_view<KIND>(NAME, dtype, x, out, w, ddof, ws, ws_bytes, stream)
+  NBG_COLS("nbg_nansum", kRSum);
+  NBG_COLS("nbg_nanmean", kRMean);
+  NBG_COLS("nbg_nancount", kRCount);
+  NBG_COLS("nbg_allnan", kRAllNan);
+  NBG_COLS("nbg_anynan", kRAnyNan);
+  NBG_COLS("nbg_nanvar", kRVar);
+  NBG_COLS("nbg_nanstd", kRStd);
+  NBG_COLS("nbg_nanmax", kRMax);
+  NBG_COLS("nbg_nanmin", kRMin);
+  NBG_COLS("nbg_nanargmax", kRArgMax);
+  NBG_COLS("nbg_nanargmin", kRArgMin);
+#undef NBG_COLS
+  return set_error(NBG_ERR_INVALID, "nbg_reduce_cols: unknown reduction %s", name);
+}
 
 size_t nbg_reduce_workspace_bytes(int64_t rows, int64_t n, int dtype) {
   const int elem = (dtype == NBG_F64 || dtype == NBG_I64) ? 8 : 4;

@@ -540,6 +540,73 @@ def _reduce_rows(t: torch.Tensor, axes: tuple[int, ...]):
     return v2, rows, n2, ld, outer
 
 
+def _inner_split(t: torch.Tensor, axes: tuple[int, ...]):
+    """(outer, n, cols, ld_outer, ld_row) of a reduction of ``t`` over ``axes``
+    that leaves its innermost axis, or None.
+
+    The dimensions are taken in memory order (largest stride first): kept ones,
+    then the reduced ones, then kept ones down to unit stride, each group in
+    the order of the result (kept) or of ``axes`` (reduced, which the indices
+    of arg* count in) and evenly strided. Everything else goes through the
+    general path, which moves the reduced axes last. So do tiny inner parts of
+    many outer entries, whose workgroups would be nearly empty.
+    """
+    dims = [d for d in range(t.dim()) if t.shape[d] != 1]
+    if t.numel() == 0 or not dims or any(t.stride(d) <= 0 for d in dims):
+        return None
+    order = sorted(dims, key=lambda d: -t.stride(d))
+    reduced = [d for d in order if d in axes]
+    if not reduced or order[-1] in axes or t.stride(order[-1]) != 1:
+        return None
+    if reduced != [a for a in axes if t.shape[a] != 1]:
+        return None
+    kept = [d for d in order if d not in axes]
+    if kept != sorted(kept):
+        return None
+    first = order.index(reduced[0])
+    groups = [order[:first], order[first:first + len(reduced)], order[first + len(reduced):]]
+    if groups[1] != reduced:
+        return None
+    sizes, steps = [], []
+    for g in groups:
+        for d, e in zip(g, g[1:]):
+            if t.stride(d) != t.shape[e] * t.stride(e):
+                return None
+        sizes.append(int(np.prod([t.shape[d] for d in g], dtype=np.int64)))
+        steps.append(int(t.stride(g[-1])) if g else 0)
+    outer, n, cols = sizes
+    if steps[1] < cols or (outer > 1 and n * cols < 512):
+        return None
+    return outer, n, cols, steps[0], steps[1]
+
+
+def _run_reduction(op: _Op, t: torch.Tensor, axes: tuple[int, ...], out_dtype, ddof=None):
+    """Launch the reduction ``op`` of ``t`` over ``axes`` into a new tensor;
+    (that tensor, flat; the result's shape)."""
+    cols = _inner_split(t, axes)
+    if cols is not None:
+        outer = tuple(t.shape[d] for d in range(t.dim()) if d not in axes)
+        n_outer, n, n_cols, ld_outer, ld_row = cols
+        out = torch.empty(n_outer * n_cols, dtype=dev.torch_dtype(out_dtype), device=t.device)
+        code = dev.nbg_code(t)
+        ws_bytes = _lib.query("nbg_reduce_cols_workspace_bytes", n_outer, n, n_cols, code)
+        ws, ws_bytes = dev.workspace(ws_bytes, t.device)
+        _lib.call("nbg_reduce_cols", op.entry.encode(), ctypes.c_int(code), dev.ptr(t), dev.ptr(out), n_outer, n,
+                  n_cols, ld_outer, ld_row, int(ddof or 0), dev.ptr(ws), ws_bytes, dev.stream_handle())
+        return out, outer
+    v2, rows, n, ld, outer = _reduce_rows(t, axes)
+    out = torch.empty(rows, dtype=dev.torch_dtype(out_dtype), device=t.device)
+    if rows:
+        ws_bytes = _lib.query("nbg_reduce_workspace_bytes", rows, n, dev.nbg_code(v2))
+        ws, ws_bytes = dev.workspace(ws_bytes, t.device)
+        args = [ctypes.c_int(dev.nbg_code(v2)), dev.ptr(v2), dev.ptr(out), rows, n, ld]
+        if ddof is not None:
+            args.append(int(ddof))
+        args += [dev.ptr(ws), ws_bytes, dev.stream_handle()]
+        _lib.call(op.entry, *args)
+    return out, outer
+
+
 def _scalar_or_array(res: torch.Tensor, outer: tuple, as_tensor: bool):
     out = dev.to_output(res.view(outer) if outer else res.view(()), as_tensor)
     if not as_tensor and not outer:
@@ -579,17 +646,7 @@ class ndaggregate(_Op):
         as_tensor = dev.is_tensor(arr)
         loop = _first_safe_loop(dev.np_dtype(arr), self.loops, self.__name__)
         t = dev.to_device(arr, loop)
-        v2, rows, n, ld, outer = _reduce_rows(t, axes)
-        odt = self.out_dtype or loop
-        out = torch.empty(rows, dtype=dev.torch_dtype(odt), device=t.device)
-        if rows:
-            ws_bytes = _lib.query("nbg_reduce_workspace_bytes", rows, n, dev.nbg_code(v2))
-            ws, ws_bytes = dev.workspace(ws_bytes, t.device)
-            args = [ctypes.c_int(dev.nbg_code(v2)), dev.ptr(v2), dev.ptr(out), rows, n, ld]
-            if self.supports_ddof:
-                args.append(int(ddof))
-            args += [dev.ptr(ws), ws_bytes, dev.stream_handle()]
-            _lib.call(self.entry, *args)
+        out, outer = _run_reduction(self, t, axes, self.out_dtype or loop, int(ddof) if self.supports_ddof else None)
         return _scalar_or_array(out, outer, as_tensor)
 
 
@@ -623,24 +680,16 @@ class ndreduce(_Op):
         as_tensor = dev.is_tensor(arr)
         loop = _first_safe_loop(dev.np_dtype(arr), self._LOOPS, self.__name__)
         t = dev.to_device(arr, loop)
-        v2, rows, n, ld, outer = _reduce_rows(t, axes)
-        if self.index:
-            odt = np.dtype(np.int64)
-        else:
-            odt = np.dtype(np.int64) if loop.kind == "i" else loop
-        out = torch.empty(rows, dtype=dev.torch_dtype(odt), device=t.device)
-        if rows and n == 0:
+        kept = [t.shape[d] for d in range(ndim) if d not in axes]
+        if 0 not in kept and any(t.shape[d] == 0 for d in axes):
             if self.index:
                 raise ValueError("All-NaN slice encountered")
             op = "fmax" if self.__name__ == "nanmax" else "fmin"
             raise ValueError(f"zero-size array to reduction operation {op} which has no identity")
-        if rows:
-            ws_bytes = _lib.query("nbg_reduce_workspace_bytes", rows, n, dev.nbg_code(v2))
-            ws, ws_bytes = dev.workspace(ws_bytes, t.device)
-            _lib.call(self.entry, ctypes.c_int(dev.nbg_code(v2)), dev.ptr(v2), dev.ptr(out), rows, n, ld,
-                      dev.ptr(ws), ws_bytes, dev.stream_handle())
-            if self.index and bool((out < 0).any().item()):
-                raise ValueError("All-NaN slice encountered")
+        odt = np.dtype(np.int64) if self.index or loop.kind == "i" else loop
+        out, outer = _run_reduction(self, t, axes, odt)
+        if self.index and out.numel() and bool((out < 0).any().item()):
+            raise ValueError("All-NaN slice encountered")
         return _scalar_or_array(out, outer, as_tensor)
 
 

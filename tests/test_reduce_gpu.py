@@ -301,3 +301,68 @@ def test_extreme_ties_signed_zeros_and_infinities(gpu_lib, func, dtype):
     want = restated.reduce(func, x)
     assert got.dtype == want.dtype
     assert_array_equal(got.view(np.uint8), want.view(np.uint8))
+
+
+REDUCERS = ["nansum", "nanmean", "nancount", "nanvar", "nanstd", "allnan", "anynan", "nanmax", "nanmin",
+            "nanargmax", "nanargmin"]
+
+
+# column counts around the 16-byte vector, the wave and the tile of columns;
+# lengths around the unrolled step, the row lanes and the row splits
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.int32, np.int64])
+@pytest.mark.parametrize("shape", [(1, 1, 5), (1, 9, 2), (3, 200, 3), (1, 1000, 63), (1, 700, 65), (2, 333, 127),
+                                   (1, 65, 128), (1, 4097, 129), (1, 300, 257), (2, 31, 1030), (1, 20_000, 7)])
+def test_inner_axis_kept(gpu_lib, shape, dtype):
+    """Reductions over an axis in front of the innermost, read as they lie
+    (also at odd element offsets), give what the same call gives on a copy
+    with that axis last: exactly for copies, counts and indices, within the
+    float bars of this file otherwise."""
+    import torch
+
+    import numbagg_amd as nb
+
+    rng = np.random.default_rng(sum(shape))
+    x = rng.integers(-50, 50, (*shape[:2], shape[2] + 1)).astype(dtype)
+    if np.issubdtype(dtype, np.floating):
+        x = (x * rng.random(x.shape)).astype(dtype)
+        x[rng.random(x.shape) < 0.1] = np.nan
+        x[:, 0] = 1.5  # no all-NaN column
+    t = torch.from_numpy(x).cuda()[:, :, 1:]
+    for name in REDUCERS:
+        f = getattr(nb, name)
+        got = f(t, axis=1)
+        want = f(t.movedim(1, -1).contiguous(), axis=-1)
+        assert got.shape == want.shape and got.dtype == want.dtype, name
+        if name in ("nanmean", "nanvar", "nanstd", "nansum") and got.is_floating_point():
+            g, w = got.cpu().numpy(), want.cpu().numpy()
+            # both sides are within one rounding (float32) or 1e-13 (float64) of the exact value
+            assert_allclose(g, w, rtol=2.4e-7 if g.dtype == np.float32 else 1e-12, atol=1e-11, err_msg=name)
+        else:
+            assert torch.equal(got, want), name
+
+
+def test_inner_axis_kept_special_values(gpu_lib):
+    """Columns of one repeated value have no variance, infinities propagate,
+    all-NaN columns give NaN (arg*: the error), ties go to the first index."""
+    import torch
+
+    import numbagg_amd as nb
+
+    x = np.full((1003, 130), 0.1, dtype=np.float32)
+    x[5::7, 1] = np.nan
+    x[:, 2] = np.nan
+    x[10, 3], x[20, 4] = np.inf, -np.inf
+    x[::2, 5] = -0.0
+    t = torch.from_numpy(x).cuda()
+    var = nb.nanvar(t, axis=0).cpu().numpy()
+    keep = np.ones(130, bool)
+    keep[2:6] = False
+    assert (var[keep] == 0).all() and np.isnan(var[2:5]).all()
+    total = nb.nansum(t, axis=0).cpu().numpy()
+    assert total[2] == 0 and total[3] == np.inf and total[4] == -np.inf
+    assert np.isnan(nb.nanmean(t, axis=0)[2].item()) and np.isnan(nb.nanmax(t, axis=0)[2].item())
+    with pytest.raises(ValueError, match="All-NaN"):
+        nb.nanargmax(t, axis=0)
+    at = nb.nanargmax(t[:, 6:], axis=0)
+    assert not at.any()
+    assert nb.nanargmin(t[:, 3:6], axis=0).tolist() == [0, 20, 0]
