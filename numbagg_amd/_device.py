@@ -9,7 +9,7 @@ torch's caching allocator, so steady-state calls never hit hipMalloc.
 
 from __future__ import annotations
 
-import ctypes
+import math
 import threading
 
 import numpy as np
@@ -51,6 +51,13 @@ def require_gpu() -> None:
         )
 
 
+# A call on a GPU tensor of the wanted dtype takes about 10 us of host time in
+# all (move_mean on a (100, 10000) array; 36 us before): the helpers below
+# keep to attribute reads, dict lookups and plain ints there. A tensor on the
+# GPU shows by itself that one is visible, so only host arrays ask torch for
+# it.
+
+
 def is_tensor(x) -> bool:
     return isinstance(x, torch.Tensor)
 
@@ -63,10 +70,12 @@ def np_dtype(x) -> np.dtype:
 
 
 def torch_dtype(dt: np.dtype) -> torch.dtype:
-    try:
-        return _NP_TO_TORCH[np.dtype(dt).newbyteorder("=")]
-    except KeyError:
-        raise TypeError(f"numbagg_amd: unsupported dtype {dt}") from None
+    td = _NP_TO_TORCH.get(dt)
+    if td is None:
+        td = _NP_TO_TORCH.get(np.dtype(dt).newbyteorder("="))
+    if td is None:
+        raise TypeError(f"numbagg_amd: unsupported dtype {dt}")
+    return td
 
 
 def nbg_code(t: torch.Tensor) -> int:
@@ -75,10 +84,13 @@ def nbg_code(t: torch.Tensor) -> int:
 
 def to_device(a, dtype: np.dtype | None = None) -> torch.Tensor:
     """A tensor on the current GPU holding ``a`` (cast to ``dtype`` if given)."""
-    require_gpu()
-    if isinstance(a, torch.Tensor):
-        t = a if a.is_cuda else a.cuda()
+    if isinstance(a, torch.Tensor) and a.is_cuda:
+        t = a
+    elif isinstance(a, torch.Tensor):
+        require_gpu()
+        t = a.cuda()
     else:
+        require_gpu()
         arr = np.asarray(a)
         if arr.dtype.byteorder not in ("=", "|"):
             arr = arr.astype(arr.dtype.newbyteorder("="))
@@ -101,7 +113,7 @@ def rows_view(t: torch.Tensor) -> tuple[torch.Tensor, int, int, int]:
     only when the outer dimensions cannot be flattened into a single stride.
     """
     n = t.shape[-1] if t.dim() else 1
-    rows = int(np.prod(t.shape[:-1], dtype=np.int64)) if t.dim() > 1 else 1
+    rows = math.prod(t.shape[:-1]) if t.dim() > 1 else 1
     if t.dim() == 1:
         t2 = t.view(1, n) if t.stride(-1) == 1 else t.contiguous().view(1, n)
     else:
@@ -117,8 +129,9 @@ def rows_view(t: torch.Tensor) -> tuple[torch.Tensor, int, int, int]:
     return t2, rows, n, ld
 
 
-def stream_handle() -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+def stream_handle() -> int:
+    """The hipStream_t of torch's current stream on the current device."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def workspace(nbytes: int, device: torch.device) -> tuple[torch.Tensor | None, int]:
@@ -127,8 +140,8 @@ def workspace(nbytes: int, device: torch.device) -> tuple[torch.Tensor | None, i
     return torch.empty(int(nbytes), dtype=torch.uint8, device=device), int(nbytes)
 
 
-def ptr(t: torch.Tensor | None) -> ctypes.c_void_p:
-    return ctypes.c_void_p(t.data_ptr() if t is not None else 0)
+def ptr(t: torch.Tensor | None) -> int | None:
+    return t.data_ptr() if t is not None else None
 
 
 _spin_lock = threading.Lock()

@@ -180,14 +180,13 @@ def last_error() -> str:
 
 def call(name: str, *args) -> None:
     """Call an NBG entry point and raise ``RuntimeError`` on a non-zero status."""
-    fn = getattr(load(), name)
-    rc = fn(*args)
+    rc = getattr(_lib or load(), name)(*args)
     if rc != 0:
         raise RuntimeError(f"{name} failed (status {rc}): {last_error()}")
 
 
 def query(name: str, *args) -> int:
-    return int(getattr(load(), name)(*args))
+    return getattr(_lib or load(), name)(*args)
 
 
 def spin_timeouts() -> int:

@@ -12,10 +12,10 @@ bodies are never executed. There is no CPU fallback.
 
 from __future__ import annotations
 
-import ctypes
 import functools
 import inspect
 import logging
+import math
 import os
 from collections.abc import Callable
 from typing import Any
@@ -31,13 +31,20 @@ from . import plain_tuning
 logger = logging.getLogger(__name__)
 
 
+_F32, _F64 = np.dtype(np.float32), np.dtype(np.float64)
+
+
 def _loop_dtype(dtypes: list[np.dtype], func_name: str) -> np.dtype:
     """The float loop NumPy's gufunc type resolution would pick.
 
     numbagg registers a float32 loop then a float64 loop (e.g. moving.py:12-14);
     NumPy takes the first loop every operand can be cast to safely.
     """
-    for loop in (np.dtype(np.float32), np.dtype(np.float64)):
+    if all(dt is _F32 for dt in dtypes):
+        return _F32
+    if all(dt is _F64 for dt in dtypes):
+        return _F64
+    for loop in (_F32, _F64):
         if all(np.can_cast(dt, loop, casting="safe") for dt in dtypes):
             return loop
     raise TypeError(
@@ -139,8 +146,10 @@ def _broadcast_rows(tensors: list[torch.Tensor], axes: list[int]):
 
     Returns (list of (rows, n) views with ld, outer_shape, n).
     """
-    moved = [t.movedim(ax, -1) for t, ax in zip(tensors, axes)]
+    moved = [t if ax == -1 else t.movedim(ax, -1) for t, ax in zip(tensors, axes)]
     n = moved[0].shape[-1]
+    if len(moved) == 1 or all(m.shape == moved[0].shape for m in moved):
+        return [dev.rows_view(m) for m in moved], tuple(moved[0].shape[:-1]), n
     for m in moved[1:]:
         if m.shape[-1] != n:
             raise ValueError(
@@ -198,7 +207,7 @@ class ndmove(_Op):
         rows = views[0][1]
         out = torch.empty((rows, n), dtype=dev.torch_dtype(loop), device=tensors[0].device)
         if rows and n:
-            args = [ctypes.c_int(dev.nbg_code(out))]
+            args = [dev.nbg_code(out)]
             args += [dev.ptr(v[0]) for v in views]
             args += [dev.ptr(out), rows, n]
             args += [v[3] for v in views]
@@ -206,7 +215,9 @@ class ndmove(_Op):
             with plain_tuning.applied(self.__name__, loop, rows, n, int(window)):
                 _lib.call(self.entry, *args)
         # NumPy places the output's core dimension at `axis` as well.
-        res = out.view(*outer, n).movedim(-1, axis)
+        res = out if len(outer) == 1 else out.view(*outer, n)
+        if axis != -1:
+            res = res.movedim(-1, axis)
         return self._deliver(dev.to_output(res, as_tensor), dest)
 
 
@@ -264,7 +275,7 @@ class ndmoveexp(_Op):
         rows = views[0][1]
         device = tensors[0].device
 
-        alpha_ptr, ld_alpha, alpha_scalar, alpha_keep = ctypes.c_void_p(0), 0, 0.0, None
+        alpha_ptr, ld_alpha, alpha_scalar, alpha_keep = None, 0, 0.0, None
         if alpha_mode == "scalar":
             alpha_scalar = float(np.asarray(alpha, dtype=loop))
         elif alpha_mode == "row":
@@ -287,16 +298,18 @@ class ndmoveexp(_Op):
             code_in = _lib.NBG_F32 if x_dtype == np.float32 else _lib.NBG_F64
             ws_bytes = _lib.query("nbg_move_exp_workspace_bytes", rows, n, code_in)
             ws, ws_bytes = dev.workspace(ws_bytes, device)
-            args = [ctypes.c_int(code_in), ctypes.c_int(dev.nbg_code(out))]
+            args = [code_in, dev.nbg_code(out)]
             args += [dev.ptr(v[0]) for v in views]
-            args += [alpha_ptr, ld_alpha, ctypes.c_double(alpha_scalar), dev.ptr(out), rows, n]
+            args += [alpha_ptr, ld_alpha, alpha_scalar, dev.ptr(out), rows, n]
             args += [v[3] for v in views]
-            args += [n, ctypes.c_double(mw), dev.ptr(ws), ws_bytes, dev.stream_handle()]
+            args += [n, mw, dev.ptr(ws), ws_bytes, dev.stream_handle()]
             with plain_tuning.applied(self.__name__, loop, rows, n):
                 _lib.call(self.entry, *args)
         del alpha_keep
         # NumPy places the output's core dimension at `axis` as well.
-        res = out.view(*outer, n).movedim(-1, axis)
+        res = out if len(outer) == 1 else out.view(*outer, n)
+        if axis != -1:
+            res = res.movedim(-1, axis)
         return self._deliver(dev.to_output(res, as_tensor), dest)
 
 
@@ -326,7 +339,7 @@ class ndfill(_Op):
         # float16 rows are filled through float32, which round-trips exactly.
         work = np.dtype(np.float32) if dt == np.float16 else dt
         t = dev.to_device(arr, work)
-        moved = t.movedim(axis, -1)
+        moved = t if axis == -1 else t.movedim(axis, -1)
         v2, rows, n, ld = dev.rows_view(moved)
         out = torch.empty((rows, n), dtype=t.dtype, device=t.device)
         if rows and n:
@@ -336,7 +349,7 @@ class ndfill(_Op):
                 ws, ws_bytes = dev.workspace(ws_bytes, t.device)
                 _lib.call(
                     self.entry,
-                    ctypes.c_int(dev.nbg_code(t)),
+                    dev.nbg_code(t),
                     dev.ptr(v2),
                     dev.ptr(out),
                     rows,
@@ -348,7 +361,9 @@ class ndfill(_Op):
                     ws_bytes,
                     dev.stream_handle(),
                 )
-        res = out.view(moved.shape).movedim(-1, axis)
+        res = out.view(moved.shape)
+        if axis != -1:
+            res = res.movedim(-1, axis)
         if work != dt:
             res = res.to(dev.torch_dtype(dt))
         return self._deliver(dev.to_output(res, as_tensor), dest)
@@ -457,15 +472,18 @@ class groupndreduce(_Op):
         v = dev.to_device(values, kdt)
         if v.dtype == torch.bool:
             v = v.to(torch.int32)
-        v = v.movedim(core_axes, list(range(ndim - len(core_axes), ndim)))
-        n = int(np.prod([vshape[a] for a in core_axes], dtype=np.int64))
-        rows = int(np.prod(broadcast_shape, dtype=np.int64))
+        last = list(range(ndim - len(core_axes), ndim))
+        if core_axes != last:
+            v = v.movedim(core_axes, last)
+        n = math.prod(vshape[a] for a in core_axes)
+        rows = math.prod(broadcast_shape)
         v2 = v.reshape(rows, n)
         if v2.stride(-1) != 1 or (rows > 1 and v2.stride(0) < n):
             v2 = v2.contiguous()
         ld_v = int(v2.stride(0)) if rows > 1 else n
         lab = dev.to_device(labels)
-        lab = lab.to(torch.int32 if lab.dtype in (torch.int8, torch.int16) else lab.dtype)
+        if lab.dtype in (torch.int8, torch.int16):
+            lab = lab.to(torch.int32)
         lab = lab.reshape(n).contiguous()
 
         out = torch.empty((rows, num_labels), dtype=dev.torch_dtype(kdt), device=v2.device)
@@ -476,9 +494,9 @@ class groupndreduce(_Op):
             )
             ws, ws_bytes = dev.workspace(ws_bytes, v2.device)
             args = [
-                ctypes.c_int(dev.nbg_code(v2)),
+                dev.nbg_code(v2),
                 dev.ptr(v2),
-                ctypes.c_int(dev.nbg_code(lab)),
+                dev.nbg_code(lab),
                 dev.ptr(lab),
                 dev.ptr(out),
                 rows,
@@ -488,7 +506,7 @@ class groupndreduce(_Op):
             ]
             if self.supports_ddof:
                 args.append(int(ddof))
-            args += [ctypes.c_int(strategy), dev.ptr(ws), ws_bytes, dev.stream_handle()]
+            args += [strategy, dev.ptr(ws), ws_bytes, dev.stream_handle()]
             with plain_tuning.applied(self.__name__, kdt, rows, n, int(num_labels)):
                 _lib.call(self.entry, *args)
         res = out.view(*broadcast_shape, num_labels)
@@ -519,6 +537,8 @@ class groupndreduce(_Op):
 def _first_safe_loop(dt: np.dtype, loops: list[np.dtype], func_name: str) -> np.dtype:
     """NumPy's loop choice for a gufunc with the given loops: the first one the
     input casts to safely (what numba's guvectorize registers, in order)."""
+    if dt is _F32 and _F32 in loops:  # float32 casts safely to no loop before its own
+        return _F32
     for loop in loops:
         if np.can_cast(dt, loop, casting="safe"):
             return loop
@@ -532,9 +552,10 @@ def _reduce_rows(t: torch.Tensor, axes: tuple[int, ...]):
     """Move `axes` (in that order) last and flatten them: (rows, n) view plus
     the outer shape (numbagg/utils.py:20-32)."""
     ndim = t.dim()
-    moved = t.movedim(axes, tuple(range(ndim - len(axes), ndim))) if axes else t
+    last = tuple(range(ndim - len(axes), ndim))
+    moved = t.movedim(axes, last) if axes != last else t
     outer = tuple(moved.shape[: ndim - len(axes)])
-    n = int(np.prod(moved.shape[ndim - len(axes):], dtype=np.int64))
+    n = math.prod(moved.shape[ndim - len(axes):])
     flat = moved.reshape(*outer, n) if outer else moved.reshape(n)
     v2, rows, n2, ld = dev.rows_view(flat)
     return v2, rows, n2, ld, outer
@@ -551,6 +572,15 @@ def _inner_split(t: torch.Tensor, axes: tuple[int, ...]):
     general path, which moves the reduced axes last. So do tiny inner parts of
     many outer entries, whose workgroups would be nearly empty.
     """
+    if t.is_contiguous() and t.numel():
+        if t.dim() - 1 in axes:
+            return None
+        if axes and axes == tuple(range(axes[0], axes[-1] + 1)):
+            outer, n, cols = (math.prod(t.shape[a:b]) for a, b in
+                              ((0, axes[0]), (axes[0], axes[-1] + 1), (axes[-1] + 1, t.dim())))
+            if cols == 1 or (outer > 1 and n * cols < 512):
+                return None
+            return outer, n, cols, n * cols, cols
     dims = [d for d in range(t.dim()) if t.shape[d] != 1]
     if t.numel() == 0 or not dims or any(t.stride(d) <= 0 for d in dims):
         return None
@@ -572,7 +602,7 @@ def _inner_split(t: torch.Tensor, axes: tuple[int, ...]):
         for d, e in zip(g, g[1:]):
             if t.stride(d) != t.shape[e] * t.stride(e):
                 return None
-        sizes.append(int(np.prod([t.shape[d] for d in g], dtype=np.int64)))
+        sizes.append(math.prod(t.shape[d] for d in g))
         steps.append(int(t.stride(g[-1])) if g else 0)
     outer, n, cols = sizes
     if steps[1] < cols or (outer > 1 and n * cols < 512):
@@ -591,7 +621,7 @@ def _run_reduction(op: _Op, t: torch.Tensor, axes: tuple[int, ...], out_dtype, d
         code = dev.nbg_code(t)
         ws_bytes = _lib.query("nbg_reduce_cols_workspace_bytes", n_outer, n, n_cols, code)
         ws, ws_bytes = dev.workspace(ws_bytes, t.device)
-        _lib.call("nbg_reduce_cols", op.entry.encode(), ctypes.c_int(code), dev.ptr(t), dev.ptr(out), n_outer, n,
+        _lib.call("nbg_reduce_cols", op.entry.encode(), code, dev.ptr(t), dev.ptr(out), n_outer, n,
                   n_cols, ld_outer, ld_row, int(ddof or 0), dev.ptr(ws), ws_bytes, dev.stream_handle())
         return out, outer
     v2, rows, n, ld, outer = _reduce_rows(t, axes)
@@ -599,7 +629,7 @@ def _run_reduction(op: _Op, t: torch.Tensor, axes: tuple[int, ...], out_dtype, d
     if rows:
         ws_bytes = _lib.query("nbg_reduce_workspace_bytes", rows, n, dev.nbg_code(v2))
         ws, ws_bytes = dev.workspace(ws_bytes, t.device)
-        args = [ctypes.c_int(dev.nbg_code(v2)), dev.ptr(v2), dev.ptr(out), rows, n, ld]
+        args = [dev.nbg_code(v2), dev.ptr(v2), dev.ptr(out), rows, n, ld]
         if ddof is not None:
             args.append(int(ddof))
         args += [dev.ptr(ws), ws_bytes, dev.stream_handle()]
@@ -701,7 +731,7 @@ def _matrix_loop(a, func_name: str) -> np.dtype:
 def _batched(t: torch.Tensor) -> tuple[torch.Tensor, tuple[int, ...], int]:
     """(batch, d0, d1) contiguous view of ``t`` (..., d0, d1)."""
     outer = tuple(t.shape[:-2])
-    batch = int(np.prod(outer, dtype=np.int64)) if outer else 1
+    batch = math.prod(outer)
     return t.contiguous().view(batch, t.shape[-2], t.shape[-1]), outer, batch
 
 
@@ -733,7 +763,7 @@ class ndmatrix(_Op):
             else:
                 ws_bytes = _lib.query("nbg_matrix_workspace_bytes", batch, nv, nobs)
                 ws, ws_bytes = dev.workspace(ws_bytes, t.device)
-                _lib.call(self.entry, ctypes.c_int(dev.nbg_code(out)), dev.ptr(x), dev.ptr(out), batch, nv, nobs,
+                _lib.call(self.entry, dev.nbg_code(out), dev.ptr(x), dev.ptr(out), batch, nv, nobs,
                           dev.ptr(ws), ws_bytes, dev.stream_handle())
         return self._deliver(dev.to_output(out.view(*outer, nv, nv), as_tensor), dest)
 
@@ -770,7 +800,7 @@ class ndmovematrix(_Op):
         if batch and nobs and nv:
             ws_bytes = _lib.query("nbg_move_matrix_workspace_bytes", batch, nobs, nv, int(window))
             ws, ws_bytes = dev.workspace(ws_bytes, t.device)
-            _lib.call(self.entry, ctypes.c_int(dev.nbg_code(out)), dev.ptr(x), dev.ptr(out), batch, nobs, nv,
+            _lib.call(self.entry, dev.nbg_code(out), dev.ptr(x), dev.ptr(out), batch, nobs, nv,
                       int(window), int(min_count), dev.ptr(ws), ws_bytes, dev.stream_handle())
         return self._deliver(dev.to_output(out.view(*outer, nobs, nv, nv), as_tensor), dest)
 
@@ -826,7 +856,7 @@ class ndmoveexpmatrix(_Op):
             code_in = _lib.NBG_F32 if x_dtype == np.float32 else _lib.NBG_F64
             ws_bytes = _lib.query("nbg_move_exp_matrix_workspace_bytes", batch, nobs, nv)
             ws, ws_bytes = dev.workspace(ws_bytes, t.device)
-            _lib.call(self.entry, ctypes.c_int(code_in), ctypes.c_int(dev.nbg_code(out)), dev.ptr(x),
-                      dev.ptr(alpha_t), ld_alpha, ctypes.c_double(mw), dev.ptr(out), batch, nobs, nv, dev.ptr(ws),
+            _lib.call(self.entry, code_in, dev.nbg_code(out), dev.ptr(x),
+                      dev.ptr(alpha_t), ld_alpha, mw, dev.ptr(out), batch, nobs, nv, dev.ptr(ws),
                       ws_bytes, dev.stream_handle())
         return self._deliver(dev.to_output(out.view(*outer, nobs, nv, nv), as_tensor), dest)

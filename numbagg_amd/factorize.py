@@ -11,8 +11,6 @@ appearance).
 
 from __future__ import annotations
 
-import ctypes
-
 import numpy as np
 import torch
 
@@ -46,12 +44,12 @@ def factorize(values, sort: bool = True):
     ws, ws_bytes = dev.workspace(ws_bytes, t.device)
     total = torch.zeros(1, dtype=torch.int64, device=t.device)
     stream = dev.stream_handle()
-    _lib.call("nbg_factorize_count", ctypes.c_int(code), dev.ptr(t), n, ctypes.c_int(int(sort)), dev.ptr(ws),
+    _lib.call("nbg_factorize_count", code, dev.ptr(t), n, int(sort), dev.ptr(ws),
               ws_bytes, dev.ptr(total), stream)
     k = int(total.item())  # the uniques' count sizes the output
     codes = torch.empty(n, dtype=torch.int64, device=t.device)
     uniques = torch.empty(k, dtype=t.dtype, device=t.device)
-    _lib.call("nbg_factorize_finish", ctypes.c_int(code), dev.ptr(t), n, k, ctypes.c_int(int(sort)),
+    _lib.call("nbg_factorize_finish", code, dev.ptr(t), n, k, int(sort),
               dev.ptr(codes), dev.ptr(uniques), dev.ptr(ws), ws_bytes, stream)
     if work != dt and not as_tensor:
         uniques = uniques.to(dev.torch_dtype(dt)) if dt.kind != "b" else uniques.to(torch.bool)

@@ -96,7 +96,7 @@ def _func_of(key: str) -> str:
 
 
 def _bucket(v: int) -> int:
-    return int(math.floor(math.log2(v))) if v > 0 else -1
+    return v.bit_length() - 1 if v > 0 else -1
 
 
 def shape_key(arch: str, func: str, dtype: str, rows: int, n: int, extra: int = 0) -> str:
@@ -113,6 +113,7 @@ class PlainTuningDB:
         self.path = pathlib.Path(path)
         self.versions = kernel_versions()
         self.entries: dict[str, dict] = {}
+        self._lookups: dict[tuple, dict | None] = {}  # (func, dtype, size classes) -> knobs
         self._lock = threading.Lock()
         try:
             with open(self.path) as f:
@@ -131,9 +132,21 @@ class PlainTuningDB:
         rec = self.entries.get(key)
         return None if rec is None else rec.get("knobs")
 
+    def lookup(self, func: str, dtype, rows: int, n: int, extra: int) -> dict | None:
+        """``get`` of this device's shape class, without building its key each
+        time (one entry per class seen: log2 sizes, so a few thousand at most)."""
+        at = (func, dtype, rows.bit_length(), n.bit_length(), extra.bit_length())
+        try:
+            return self._lookups[at]
+        except KeyError:
+            knobs = self.get(shape_key(device_arch(), func, str(dtype), rows, n, extra)) or None
+            self._lookups[at] = knobs
+            return knobs
+
     def put(self, key: str, knobs: dict, timings: dict) -> None:
         with self._lock:
             self.entries[key] = {"knobs": knobs, "timings_ms": timings}
+            self._lookups = {}
 
     def save(self) -> None:
         self.path.parent.mkdir(parents=True, exist_ok=True)
@@ -203,22 +216,25 @@ def knobs_set(knobs: dict):
 
 
 @contextlib.contextmanager
-def applied(func: str, dtype, rows: int, n: int, extra: int = 0):
-    """Apply the recorded setting of this call's shape class, if any (unless
-    explicit overrides are in force on this thread)."""
-    db = database()
-    if not db.entries or getattr(_local, "explicit", 0):
-        yield
-        return
-    knobs = db.get(shape_key(device_arch(), func, str(dtype), rows, n, extra))
-    if not knobs:
-        yield
-        return
+def _set_for(knobs: dict):
     set_knobs(knobs)
     try:
         yield
     finally:
         clear_knobs()
+
+
+_AS_IT_IS = contextlib.nullcontext()
+
+
+def applied(func: str, dtype, rows: int, n: int, extra: int = 0):
+    """Context in which the recorded setting of this call's shape class, if
+    any, applies (unless explicit overrides are in force on this thread)."""
+    db = database()
+    if not db.entries or getattr(_local, "explicit", 0):
+        return _AS_IT_IS
+    knobs = db.lookup(func, dtype, rows, n, extra)
+    return _set_for(knobs) if knobs else _AS_IT_IS
 
 
 def candidates(family: str) -> list[dict]:
