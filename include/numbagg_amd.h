@@ -105,6 +105,17 @@ int nbg_move_corr(int dtype, const void* a, const void* b, void* out,
                   int64_t rows, int64_t n, int64_t ld_a, int64_t ld_b,
                   int64_t ld_out, int64_t window, int64_t min_count,
                   void* stream);                       /* moving.py:223-275 */
+/* The same functions (name: the entry point above, "nbg_move_mean") over an
+ * axis that is not the innermost: position i of series (a, c) is
+ * x[a * ld_outer + i * ld_row + c], a < outer, i < n, c < cols; out is
+ * (outer * cols, n). b and its strides are read by move_cov and move_corr only.
+ * For float32 / float64 shapes where nbg_move_cols_chunk is positive. */
+int64_t nbg_move_cols_chunk(int dtype, int64_t outer, int64_t n, int64_t cols, int64_t window);
+int nbg_move_cols(const char* name, int dtype, const void* a, const void* b,
+                  void* out, int64_t outer, int64_t n, int64_t cols,
+                  int64_t lda_outer, int64_t lda_row, int64_t ldb_outer,
+                  int64_t ldb_row, int64_t window, int64_t min_count,
+                  void* stream);
 
 /* ---- exponentially weighted windows (numbagg/moving_exp.py:12-335;
  *      ndmoveexp.__call__ at numbagg/decorators.py:374-414) --------------- */

@@ -53,6 +53,12 @@ for _name in ("nbg_move_sum", "nbg_move_mean", "nbg_move_std", "nbg_move_var"):
     _SIGNATURES[_name] = _MOVE1
 for _name in ("nbg_move_cov", "nbg_move_corr"):
     _SIGNATURES[_name] = _MOVE2
+_SIGNATURES["nbg_move_cols_chunk"] = (_c_i64, [_c_int, _c_i64, _c_i64, _c_i64, _c_i64])
+_SIGNATURES["nbg_move_cols"] = (
+    _c_int,
+    [ctypes.c_char_p, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
+     _c_i64, _c_ptr],
+)
 _SIGNATURES["nbg_move_exp_workspace_bytes"] = (_c_size, [_c_i64, _c_i64, _c_int])
 _EXP1 = (
     _c_int,

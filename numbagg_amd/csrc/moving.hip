@@ -119,14 +119,6 @@ int move_launch(const T* a, const T* b, T* out, int64_t rows, int64_t n, int64_t
                                                      min_count, s);
 }
 
-// NBG_F32_ACCUMULATOR=twosum selects FP32 TwoSum accumulators for float32
-// sum/mean instead of float64 (the float64 default is both more precise and
-// cheaper on CDNA4, where a float64 add issues at the float32 rate).
-bool f32_twosum_requested() {
-  const char* v = getenv("NBG_F32_ACCUMULATOR");
-  return v != nullptr && strcmp(v, "twosum") == 0;
-}
-
 template <int KIND>
 int move_entry(const char* name, int dtype, const void* a, const void* b, void* out, int64_t rows,
                int64_t n, int64_t ld_a, int64_t ld_b, int64_t ld_out, int64_t window,

@@ -4,6 +4,7 @@
 #pragma once
 
 #include <cstdlib>
+#include <cstring>
 #include <type_traits>
 
 #include "common.hpp"
@@ -847,6 +848,14 @@ __device__ __forceinline__ void fill_moment_lut(double* rc, int64_t window) {
 // launches read the same setting, so their tiles stay identical.
 inline int f32_sum_items() {
   return knob("NBG_MOVE_ITEMS", 16) == 32 ? 32 : 16;
+}
+
+// NBG_F32_ACCUMULATOR=twosum selects FP32 TwoSum accumulators for float32
+// sum/mean instead of float64 (the float64 default is both more precise and
+// cheaper on CDNA4, where a float64 add issues at the float32 rate).
+inline bool f32_twosum_requested() {
+  const char* v = getenv("NBG_F32_ACCUMULATOR");
+  return v != nullptr && strcmp(v, "twosum") == 0;
 }
 
 // Whether a float32 mean of this window uses the table (plain and ragged

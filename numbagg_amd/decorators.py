@@ -203,6 +203,9 @@ class ndmove(_Op):
         as_tensor = any(dev.is_tensor(a) for a in arr)
         loop = _loop_dtype([dev.np_dtype(a) for a in arr], self.__name__)
         tensors = [dev.to_device(a, loop) for a in arr]
+        out = self._along_columns(tensors, axis, int(window), int(min_count)) if axis != -1 else None
+        if out is not None:
+            return self._deliver(dev.to_output(out, as_tensor), dest)
         views, outer, n = _broadcast_rows(tensors, [axis] * len(tensors))
         rows = views[0][1]
         out = torch.empty((rows, n), dtype=dev.torch_dtype(loop), device=tensors[0].device)
@@ -219,6 +222,28 @@ class ndmove(_Op):
         if axis != -1:
             res = res.movedim(-1, axis)
         return self._deliver(dev.to_output(res, as_tensor), dest)
+
+
+    def _along_columns(self, tensors: list[torch.Tensor], axis: int, window: int, min_count: int):
+        """The result over an axis in front of the innermost, read as it lies,
+        or None where the general path runs (other layouts, broadcast inputs,
+        few columns, long windows)."""
+        first = tensors[0]
+        if any(t.shape != first.shape for t in tensors):
+            return None
+        axis = axis % first.dim()
+        plans = [_inner_split(t, (axis,)) for t in tensors]
+        if None in plans or any(p[:3] != plans[0][:3] for p in plans):
+            return None
+        outer, n, cols = plans[0][:3]
+        code = dev.nbg_code(first)
+        if _lib.query("nbg_move_cols_chunk", code, outer, n, cols, window) == 0:
+            return None
+        kept = [s for d, s in enumerate(first.shape) if d != axis]
+        out = torch.empty((*kept, n), dtype=first.dtype, device=first.device)
+        _lib.call("nbg_move_cols", self.entry.encode(), code, dev.ptr(first), dev.ptr(tensors[-1]), dev.ptr(out),
+                  outer, n, cols, *plans[0][3:], *plans[-1][3:], window, min_count, dev.stream_handle())
+        return out.movedim(-1, axis)
 
 
 class ndmoveexp(_Op):

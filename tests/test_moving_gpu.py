@@ -274,3 +274,95 @@ def test_element_aligned_rows_match_contiguous(gpu_lib, func):
     got = getattr(nb, func)(*args_v, window=1000, min_count=500)
     want = getattr(nb, func)(*args_c, window=1000, min_count=500)
     assert torch.equal(got.view(torch.int32), want.view(torch.int32))
+
+
+# column counts around the wave, lengths around the 32-position tile and the
+# ranges of positions, windows from 1 to the longest the kernel takes
+@pytest.mark.parametrize("func", FUNCS1 + FUNCS2)
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("shape,window,min_count", [
+    ((1, 33, 32), 1, 0), ((2, 64, 64), 7, None), ((1, 200, 65), 64, 10), ((3, 129, 130), 128, 1),
+    ((1, 1000, 33), 5, 2), ((1, 31, 200), 31, 4), ((2, 3000, 40), 100, 50)])
+def test_move_inner_axis_kept(gpu_lib, func, dtype, shape, window, min_count):
+    """Windows along an axis in front of the innermost (read as it lies, also
+    at odd element offsets) against the exact oracle, with the bars above."""
+    import torch
+
+    import numbagg_amd as nb
+    from numbagg_amd import _lib
+    from oracle import exact
+
+    code = _lib.NBG_F32 if dtype == np.float32 else _lib.NBG_F64
+    assert _lib.query("nbg_move_cols_chunk", code, *shape, window) > 0
+    full = [walk_array(shape[0] * (shape[2] + 1), shape[1], seed=s + shape[1], dtype=dtype)
+            .reshape(shape[0], shape[2] + 1, shape[1]) for s in range(2 if func in FUNCS2 else 1)]
+    rows = [np.ascontiguousarray(x[:, 1:]).reshape(-1, shape[1]) for x in full]
+    tens = [torch.from_numpy(np.ascontiguousarray(x.transpose(0, 2, 1))).cuda()[:, :, 1:] for x in full]
+    got = getattr(nb, func)(*tens, window=window, min_count=min_count, axis=1)
+    assert tuple(got.shape) == shape
+    assert got.movedim(1, -1).is_contiguous()  # the layout of the general path
+    got = got.movedim(1, -1).reshape(-1, shape[1]).cpu().numpy()
+    want = exact.move(func, rows[0], window, min_count, y=rows[1] if func in FUNCS2 else None)
+    if dtype == np.float32:
+        check_f32(func, got, want, scale=np.ones_like(want))
+        return
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    ok = ~np.isnan(want)
+    assert_allclose(got[ok], want[ok], rtol=1e-11, atol=1e-13)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_move_inner_axis_kept_infinities(gpu_lib, dtype):
+    """An infinity shows in the windows that hold it and in no later one."""
+    import torch
+
+    import numbagg_amd as nb
+
+    rng = np.random.default_rng(3)
+    x = rng.standard_normal((300, 70)).astype(dtype)
+    x[50, 3], x[52, 3], x[100, 4] = np.inf, np.inf, -np.inf
+    t = torch.from_numpy(x).cuda()
+    s = nb.move_sum(t, window=10, min_count=1, axis=0).cpu().numpy()
+    v = nb.move_var(t, window=10, min_count=2, axis=0).cpu().numpy()
+    assert (s[50:62, 3] == np.inf).all() and (s[100:110, 4] == -np.inf).all()
+    hit = np.zeros(x.shape, bool)
+    hit[50:62, 3] = hit[100:110, 4] = True
+    assert np.isfinite(s[~hit]).all()
+    assert np.isnan(v[hit]).all() and np.isfinite(v[1:][~hit[1:]]).all()
+
+
+def test_move_inner_axis_kept_falls_back(gpu_lib):
+    """Few columns, long windows, broadcast operands and unlike layouts run on
+    the general path, with the same results."""
+    import torch
+
+    import numbagg_amd as nb
+
+    x = torch.from_numpy(walk_array(3000, 48, seed=1)).cuda()
+    y = torch.from_numpy(walk_array(48, 3000, seed=2)).cuda().t()
+    for a, kw in (((x[:, :5],), dict(window=9)), ((x,), dict(window=1500, min_count=3))):
+        want = nb.move_mean(a[0].t().contiguous(), axis=-1, **kw).t()
+        assert torch.equal(nb.move_mean(*a, axis=0, **kw).nan_to_num(), want.nan_to_num())
+    got = nb.move_cov(x, y, window=20, axis=0)
+    want = nb.move_cov(x.t().contiguous(), y.t(), window=20, axis=-1).t()
+    assert torch.equal(got.nan_to_num(), want.nan_to_num())
+
+
+@pytest.mark.parametrize("dtype,n,cols", [(np.float32, 1021, 33_003), (np.float64, 517, 33_001)])
+def test_move_inner_axis_kept_large_output(gpu_lib, dtype, n, cols):
+    """Outputs over 128 MB leave line by line, at every offset of a series
+    within its line: equal to the general path on a transposed copy up to one
+    rounding of each (means of data around 1e4)."""
+    import torch
+
+    import numbagg_amd as nb
+
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x = torch.randn(n, cols, generator=g, device="cuda", dtype=torch.float32 if dtype == np.float32 else torch.float64)
+    x += 1e4
+    x[torch.rand(n, cols, generator=g, device="cuda") < 0.1] = float("nan")
+    got = nb.move_mean(x, window=30, min_count=20, axis=0).movedim(0, -1)
+    want = nb.move_mean(x.t().contiguous(), window=30, min_count=20)
+    assert torch.equal(got.isnan(), want.isnan())
+    off = ((got - want).abs() / want.abs()).nan_to_num_(nan=0.0).max().item()
+    assert off <= (1.2e-7 if dtype == np.float32 else 4.5e-16)
