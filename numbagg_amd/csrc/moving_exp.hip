@@ -22,11 +22,12 @@
 //   * each thread re-runs its K positions from its exact incoming state, one
 //     fused multiply-add per state component (state = decay * state +
 //     contribution);
-//   * on request (NBG_EXP_TWO_PASS=1) the same tile code runs in two passes
-//     instead: independent tiles write their
-//     aggregate maps, one workgroup per row scans them into each tile's
-//     incoming state, and independent tiles re-run their positions from it
-//     (the input is read twice, but no tile waits on another).
+//   * for few rows (exp_two_pass) the same tile code runs in two passes
+//     instead: independent tiles write their aggregate maps, a scan over them
+//     gives each tile's incoming state, and independent tiles re-run their
+//     positions from it (the input is read twice, but no tile waits on
+//     another);
+//   * a scalar alpha (the usual call) has a kernel of its own, exp_uni_kernel.
 // Squares and cross products of float32 inputs are formed in float64 (exact),
 // where the reference rounds them to float32 first; the moment kinds shift
 // each row by its first finite value, so data far from zero (a random walk
@@ -272,10 +273,19 @@ constexpr int exp_items() {
   return (sizeof(TX) == 4 && ExpSpec<KIND>::NS <= 3) ? 32 : 64 / (int)sizeof(TX);
 }
 
+// Positions per thread of exp_uni_kernel: its var / std states are small enough
+// for twice the positions (float32 (256, 2M) nanvar 16 -> 32 positions 1463 ->
+// 1328 us, float64 (200, 300k) 8 -> 16 260 -> 237 us; corr 680 -> 782 and 402 ->
+// 473 us, mean of float64 unchanged).
+template <typename TX, int KIND>
+constexpr int uni_items() {
+  return (KIND == kEVar || KIND == kEStd) ? 128 / (int)sizeof(TX) : exp_items<TX, KIND>();
+}
+
 struct ExpArgs {
   const void* xa;
   const void* xb;
-  const void* alpha;  // nullptr: scalar alpha
+  const void* alpha;  // nullptr: scalar alpha (exp_uni_kernel)
   int64_t ld_alpha;   // 0: one alpha row shared by all rows
   double alpha_scalar;
   void* out;
@@ -286,14 +296,110 @@ struct ExpArgs {
   unsigned int* counters;
   double* payload;
   unsigned int* timeouts;
+  // scalar alpha: d = 1 - alpha, its square, and d^(K 2^i), the decay over 2^i
+  // threads' positions, i = 0..7 (7: half a tile), d^TILE
+  double d, d2, pw[8], ptile;
 };
+
+// Stage tile tk of a row in LDS (coalesced across the workgroup; NaN past the
+// row end).
+template <typename TX, int NARGS, int TILE>
+__device__ __forceinline__ void exp_stage(const TX* ra, const TX* rb, int64_t n, int64_t tk, TX* la, TX* lb) {
+  constexpr int VEC = 16 / (int)sizeof(TX);
+  const int tid = threadIdx.x;
+  const int64_t q0 = tk * TILE;
+  if (q0 + TILE <= n) {
+    // 16-byte accesses need element alignment only, so rows of any length and
+    // offset take them (float32
+    // nancount of (217, 227469): 244 -> 139 us)
+    struct V { TX v[VEC]; };
+    for (int e = tid * VEC; e < TILE; e += kExpThreads * VEC) {
+      V va = load_stream(reinterpret_cast<const V*>(ra + q0 + e));
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) la[pad16(e + v)] = va.v[v];
+      if (NARGS == 2) {
+        V vb = load_stream(reinterpret_cast<const V*>(rb + q0 + e));
+#pragma unroll
+        for (int v = 0; v < VEC; ++v) lb[pad16(e + v)] = vb.v[v];
+      }
+    }
+  } else {
+    for (int e = tid; e < TILE; e += kExpThreads) {
+      const int64_t p = q0 + e;
+      la[pad16(e)] = p < n ? ra[p] : canonical_nan<TX>();
+      if (NARGS == 2) lb[pad16(e)] = p < n ? rb[p] : canonical_nan<TX>();
+    }
+  }
+}
+
+// The row's shift for the moment kinds: its first finite value among its
+// first 64 positions (0 if there is none), the same in every wave.
+template <typename TX>
+__device__ __forceinline__ double exp_shift(const TX* row, int64_t n) {
+  const int ln = lane_id();
+  const double v = ln < n ? (double)row[ln] : 0.0;
+  const unsigned long long m = __ballot(ln < n && isfinite(v));
+  return m != 0ull ? read_lane(v, __ffsll((long long)m) - 1) : 0.0;
+}
+
+// A tile's outputs, K per thread. smem_raw holds the staged inputs, which every
+// thread has read for the last time when it calls this.
+template <typename TX, typename TA, int NARGS, int K>
+__device__ __forceinline__ void exp_store(const TA (&res)[K], TA* ro, int64_t t0, int64_t n, bool full,
+                                          unsigned char* smem_raw) {
+  constexpr int TILE = kExpThreads * K;
+  const int tid = threadIdx.x;
+  const int64_t e0 = (int64_t)tid * K;
+  constexpr int OV = 16 / (int)sizeof(TA);  // outputs per 16-byte store
+  // A full tile's outputs go through LDS (the staged inputs' region, free once
+  // every thread has re-run its positions), so that each store instruction
+  // writes consecutive 16-byte pieces across the wave instead of one piece
+  // per K * sizeof(TA) bytes. Rounds of XR threads' outputs fit the region;
+  // a thread's K outputs sit at stride K + 1 (conflict-free LDS writes).
+  constexpr int64_t kRegion = ((int64_t)TILE + TILE / 16 + 16) * (int64_t)sizeof(TX) * NARGS;  // pad16(TILE) + 16 slots
+  constexpr int kFit = (int)(kRegion / ((K + 1) * (int64_t)sizeof(TA)));
+  constexpr int XR = kFit >= kExpThreads ? kExpThreads : (kFit >= kExpThreads / 2 ? kExpThreads / 2 : kExpThreads / 4);
+  static_assert((int64_t)XR * (K + 1) * (int64_t)sizeof(TA) <= kRegion, "output round fits the staged region");
+  static_assert(K % OV == 0, "whole 16-byte pieces per thread");
+  if (full) {
+    TA* lo = reinterpret_cast<TA*>(smem_raw);
+    char* rot = reinterpret_cast<char*>(ro + t0);
+    struct V { TA v[OV]; };
+    __syncthreads();  // every re-run read of the staged inputs is done
+#pragma unroll
+    for (int r = 0; r < kExpThreads / XR; ++r) {
+      if (r > 0) __syncthreads();  // the previous round's reads are done
+      if (tid / XR == r) {
+        const int b = (tid - r * XR) * (K + 1);
+#pragma unroll
+        for (int j = 0; j < K; ++j) lo[b + j] = res[j];
+      }
+      __syncthreads();
+      // pieces of OV outputs: piece q of the round is thread q / (K / OV)'s
+      // outputs (q % (K / OV)) * OV ..
+      constexpr int kPieces = XR * K / OV;
+#pragma unroll
+      for (int q = tid; q < kPieces; q += kExpThreads) {
+        const int th = q / (K / OV), jo = (q % (K / OV)) * OV;
+        V vo;
+#pragma unroll
+        for (int v = 0; v < OV; ++v) vo.v[v] = lo[th * (K + 1) + jo + v];
+        store_stream16(reinterpret_cast<TA*>(rot + ((uint32_t)(r * XR * K + q * OV) * (uint32_t)sizeof(TA))), vo.v);
+      }
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < K; ++j)
+      if (t0 + e0 + j < n) ro[t0 + e0 + j] = res[j];
+  }
+}
 
 // MODE 0: one pass, incoming states by decoupled look-back. MODE 1: aggregate
 // pass (each tile's aggregate map to the payload, no outputs). MODE 2: apply
 // pass (each tile's incoming state read from the payload, where
 // exp_carry_kernel put it). Modes 1 and 2 process tiles in row-major order on
 // XCD-consecutive workgroups and never wait.
-template <typename TX, typename TA, int KIND, bool SCALAR, int MODE = 0>
+template <typename TX, typename TA, int KIND, int MODE = 0>
 __global__ __launch_bounds__(kExpThreads) void exp_kernel(ExpArgs A) {
   using Sp = ExpSpec<KIND>;
   constexpr int NS = Sp::NS;
@@ -315,39 +421,13 @@ __global__ __launch_bounds__(kExpThreads) void exp_kernel(ExpArgs A) {
                                 : (int64_t)(v_id / (uint64_t)A.tiles_per_row);
   const TX* ra = xa + row * A.ld_a;
   const TX* rb = (Sp::NARGS == 2) ? xb + row * A.ld_b : nullptr;
-  const TA* rl = al ? al + row * A.ld_alpha : nullptr;
+  const TA* rl = al + row * A.ld_alpha;
   TA* ro = out + row * A.ld_out;
   const int tid = threadIdx.x;
   const int64_t n = A.n;
   TX* la = reinterpret_cast<TX*>(smem_raw);
   TX* lb = la + pad16(TILE) + 16;
-  constexpr int VEC = 16 / (int)sizeof(TX);
-
-  // Stage tile tk in LDS (coalesced across the block; NaN past the row end).
-  auto stage = [&](int64_t tk) {
-    const int64_t q0 = tk * TILE;
-    const bool q_vec = (q0 + TILE <= n) && (((uintptr_t)(ra + q0)) % 16 == 0) &&
-                       (Sp::NARGS == 1 || ((uintptr_t)(rb + q0)) % 16 == 0);
-    if (q_vec) {
-      struct alignas(16) V { TX v[VEC]; };
-      for (int e = tid * VEC; e < TILE; e += kExpThreads * VEC) {
-        V va = load_stream(reinterpret_cast<const V*>(ra + q0 + e));
-#pragma unroll
-        for (int v = 0; v < VEC; ++v) la[pad16(e + v)] = va.v[v];
-        if (Sp::NARGS == 2) {
-          V vb = load_stream(reinterpret_cast<const V*>(rb + q0 + e));
-#pragma unroll
-          for (int v = 0; v < VEC; ++v) lb[pad16(e + v)] = vb.v[v];
-        }
-      }
-    } else {
-      for (int e = tid; e < TILE; e += kExpThreads) {
-        const int64_t p = q0 + e;
-        la[pad16(e)] = p < n ? ra[p] : canonical_nan<TX>();
-        if (Sp::NARGS == 2) lb[pad16(e)] = p < n ? rb[p] : canonical_nan<TX>();
-      }
-    }
-  };
+  auto stage = [&](int64_t tk) { exp_stage<TX, Sp::NARGS, TILE>(ra, rb, n, tk, la, lb); };
   // Blocks of a row are dispatched in order, so the ticket is almost always
   // blockIdx / rows: that tile is staged while the ticket atomic is in flight
   // and restaged only when the ticket differs.
@@ -382,22 +462,10 @@ __global__ __launch_bounds__(kExpThreads) void exp_kernel(ExpArgs A) {
   // common shift. For float32 data x - ka is exact in float64.
   double ka = 0.0, kb = 0.0;
   if constexpr (KIND == kEVar || KIND == kEStd || KIND == kECov || KIND == kECorr) {
-    const int ln = lane_id();
-    const double va = ln < n ? (double)ra[ln] : 0.0;
-    const unsigned long long ma = __ballot(ln < n && isfinite(va));
-    if (ma != 0ull) ka = read_lane(va, __ffsll((long long)ma) - 1);
-    if constexpr (Sp::NARGS == 2) {
-      const double vb = ln < n ? (double)rb[ln] : 0.0;
-      const unsigned long long mb = __ballot(ln < n && isfinite(vb));
-      if (mb != 0ull) kb = read_lane(vb, __ffsll((long long)mb) - 1);
-    }
+    ka = exp_shift(ra, n);
+    if constexpr (Sp::NARGS == 2) kb = exp_shift(rb, n);
   }
-  // SCALAR: one alpha for every position (kernel-uniform decay factors).
-  const double alpha_s = (double)(TA)A.alpha_scalar;
-  auto alpha_at = [&](int64_t p) -> double {
-    if constexpr (SCALAR) return alpha_s;
-    else return (double)rl[p];
-  };
+  auto alpha_at = [&](int64_t p) -> double { return (double)rl[p]; };
 
   // 1. this thread's map.
   Map<NS> m;
@@ -652,59 +720,537 @@ __global__ __launch_bounds__(kExpThreads) void exp_kernel(ExpArgs A) {
   } else {
     for (int j = 0; j < K && t0 + e0 + j < n; ++j) rerun(j);
   }
-  constexpr int OV = 16 / (int)sizeof(TA);  // outputs per 16-byte store
-  // A full tile's outputs go through LDS (the staged inputs' region, free once
-  // every thread has re-run its positions), so that each store instruction
-  // writes consecutive 16-byte pieces across the wave instead of one piece
-  // per K * sizeof(TA) bytes. Rounds of XR threads' outputs fit the region;
-  // a thread's K outputs sit at stride K + 1 (conflict-free LDS writes).
-  constexpr int64_t kRegion = ((int64_t)TILE + TILE / 16 + 16) * (int64_t)sizeof(TX) * Sp::NARGS;  // pad16(TILE) + 16 slots
-  constexpr int kFit = (int)(kRegion / ((K + 1) * (int64_t)sizeof(TA)));
-  constexpr int XR = kFit >= kExpThreads ? kExpThreads : (kFit >= kExpThreads / 2 ? kExpThreads / 2 : kExpThreads / 4);
-  static_assert((int64_t)XR * (K + 1) * (int64_t)sizeof(TA) <= kRegion, "output round fits the staged region");
-  static_assert(K % OV == 0, "whole 16-byte pieces per thread");
-  if (full && ((uintptr_t)(ro + t0)) % 16 == 0) {
-    TA* lo = reinterpret_cast<TA*>(smem_raw);
-    char* rot = reinterpret_cast<char*>(ro + t0);
-    struct alignas(16) V { TA v[OV]; };
-    __syncthreads();  // every re-run read of the staged inputs is done
-#pragma unroll
-    for (int r = 0; r < kExpThreads / XR; ++r) {
-      if (r > 0) __syncthreads();  // the previous round's reads are done
-      if (tid / XR == r) {
-        const int b = (tid - r * XR) * (K + 1);
-#pragma unroll
-        for (int j = 0; j < K; ++j) lo[b + j] = res[j];
-      }
-      __syncthreads();
-      // pieces of OV outputs: piece q of the round is thread q / (K / OV)'s
-      // outputs (q % (K / OV)) * OV ..
-      constexpr int kPieces = XR * K / OV;
-#pragma unroll
-      for (int q = tid; q < kPieces; q += kExpThreads) {
-        const int th = q / (K / OV), jo = (q % (K / OV)) * OV;
-        V vo;
-#pragma unroll
-        for (int v = 0; v < OV; ++v) vo.v[v] = lo[th * (K + 1) + jo + v];
-        store_stream16(reinterpret_cast<TA*>(rot + ((uint32_t)(r * XR * K + q * OV) * (uint32_t)sizeof(TA))), vo.v);
-      }
+  exp_store<TX, TA, Sp::NARGS, K>(res, ro, t0, n, full, smem_raw);
+}
+
+// ---------------------------------------------------------------------------
+// One alpha for every position (the usual call). The decays are constants of
+// the launch, so a chunk's map is its state alone: the scans move and multiply
+// NS components by powers of d and carry no products. Where the weight test
+// cannot fail (min_weight <= 0 and alpha within [0, 1]) the weight, alpha times
+// sum_weight, is not carried either.
+//
+// Bound by float64 arithmetic for the moment kinds, by HBM for the others.
+// Measured on MI355X for float32 (256, 2M), alpha 0.01 -> float64: nanvar
+// 1.33 ms (6.1 GB: 4.6 TB/s; 66 VALU instructions per position at 16 positions
+// per thread), 2.39 ms in the general kernel with its alpha fixed.
+// ---------------------------------------------------------------------------
+template <int KIND, bool WT>
+struct UniSpec {
+  // count: count; mean: numer, denom; sum: numer; var/std: sum_x2, sum_x, sum_w,
+  // sum_w2; cov: s1, s2, s12, sw, sw2; corr: those, s11, s22; then the weight
+  static constexpr int BASE = KIND == kEMean                       ? 2
+                              : KIND == kECount || KIND == kESum   ? 1
+                              : KIND == kEVar || KIND == kEStd     ? 4
+                              : KIND == kECov                      ? 5
+                                                                   : 7;
+  static constexpr int NS = BASE + (WT ? 1 : 0);
+  static constexpr int SW2 = ExpSpec<KIND>::SW2;
+  static constexpr int NARGS = ExpSpec<KIND>::NARGS;
+  static constexpr bool MOM = KIND == kEVar || KIND == kEStd || KIND == kECov || KIND == kECorr;
+  static constexpr bool SEEN = MOM || KIND == kESum;
+};
+
+// seen: valid observations, saturating at 2 (bits 0-1), and what an infinity
+// among them left in the sums for good: kInfPlus, kInfMinus or both (NaN).
+// Across chunks only these bits carry it (the sums are then finite), as a decay
+// that underflows to 0 would turn an infinity into NaN.
+template <int NS>
+struct UState {
+  double b[NS];
+  int seen;
+};
+constexpr int kInfPlus = 4, kInfMinus = 8, kInfBoth = 12;
+
+__device__ __forceinline__ int join_seen(int a, int b) {
+  return min(2, (a & 3) + (b & 3)) | ((a | b) & kInfBoth);
+}
+
+// Infinities and NaN of a chunk's sums (components 0 and, for the moment kinds,
+// all sums of observations) moved into its bits.
+template <int KIND, int NS>
+__device__ __forceinline__ void park_inf(UState<NS>& s) {
+  constexpr bool MOM = KIND >= kEVar;
+  if constexpr (KIND == kECount) return;
+  if constexpr (!MOM) {
+    if (__builtin_expect(!isfinite(s.b[0]), 0)) {
+      s.seen |= s.b[0] > 0 ? kInfPlus : (s.b[0] < 0 ? kInfMinus : kInfBoth);
+      s.b[0] = 0.0;
     }
-  } else if (full && ((uintptr_t)(ro + t0 + e0)) % 16 == 0) {
-    struct alignas(16) V { TA v[OV]; };
-#pragma unroll
-    for (int j = 0; j < K; j += OV) {
-      V vo;
-#pragma unroll
-      for (int v = 0; v < OV; ++v) vo.v[v] = res[j + v];
-      *reinterpret_cast<V*>(ro + t0 + e0 + j) = vo;
-    }
-  } else if (full) {
-#pragma unroll
-    for (int j = 0; j < K; ++j) ro[t0 + e0 + j] = res[j];
   } else {
+    bool ok = true;
 #pragma unroll
-    for (int j = 0; j < K; ++j)
-      if (t0 + e0 + j < n) ro[t0 + e0 + j] = res[j];
+    for (int c = 0; c < NS; ++c) ok = ok && isfinite(s.b[c]);
+    if (__builtin_expect(!ok, 0)) {
+      s.seen |= kInfBoth;
+#pragma unroll
+      for (int c = 0; c < NS; ++c) s.b[c] = isfinite(s.b[c]) ? s.b[c] : 0.0;
+    }
+  }
+}
+// The sums as the recurrence would hold them.
+template <int KIND, int NS>
+__device__ __forceinline__ void unpark_inf(UState<NS>& s) {
+  constexpr bool MOM = KIND >= kEVar;
+  if (KIND == kECount || __builtin_expect((s.seen & kInfBoth) == 0, 1)) return;
+  const double v = (s.seen & kInfBoth) == kInfPlus    ? __builtin_inf()
+                   : (s.seen & kInfBoth) == kInfMinus ? -__builtin_inf()
+                                                      : __builtin_nan("");
+  s.b[0] = MOM ? __builtin_nan("") : v;
+  if constexpr (MOM) {
+    s.b[1] = __builtin_nan("");
+    if constexpr (KIND == kECov || KIND == kECorr) s.b[2] = __builtin_nan("");
+  }
+  s.seen &= 3;
+}
+
+// later after `earlier` decayed over later's positions (q = d^positions).
+template <int NS, int SW2>
+__device__ __forceinline__ UState<NS> uni_join(const UState<NS>& earlier, const UState<NS>& later, double q) {
+  UState<NS> r;
+#pragma unroll
+  for (int c = 0; c < NS; ++c) r.b[c] = fma(c == SW2 ? q * q : q, earlier.b[c], later.b[c]);
+  r.seen = join_seen(earlier.seen, later.seen);
+  return r;
+}
+template <int CTRL, int RM, int NS>
+__device__ __forceinline__ UState<NS> uni_dpp(const UState<NS>& m) {
+  UState<NS> r;
+#pragma unroll
+  for (int c = 0; c < NS; ++c) r.b[c] = dpp_move<CTRL, RM>(0.0, m.b[c]);
+  r.seen = dpp_move<CTRL, RM>(0, m.seen);
+  return r;
+}
+
+// One step: ya, yb are the shifted observations (0 where invalid).
+template <int KIND, bool WT>
+__device__ __forceinline__ void uni_step(UState<UniSpec<KIND, WT>::NS>& s, bool valid, double ya, double yb, double d,
+                                         double d2, double alpha) {
+  using Sp = UniSpec<KIND, WT>;
+  const double v = valid ? 1.0 : 0.0;
+  if (Sp::SEEN) s.seen += (int)valid;
+  if constexpr (KIND == kECount) {
+    s.b[0] = fma(d, s.b[0], v);
+  } else if constexpr (KIND == kEMean) {
+    s.b[0] = fma(d, s.b[0], ya);
+    s.b[1] = fma(d, s.b[1], v);
+  } else if constexpr (KIND == kESum) {
+    s.b[0] = fma(d, s.b[0], ya);
+  } else if constexpr (KIND == kEVar || KIND == kEStd) {
+    s.b[0] = fma(d, s.b[0], ya * ya);
+    s.b[1] = fma(d, s.b[1], ya);
+    s.b[2] = fma(d, s.b[2], v);
+    s.b[3] = fma(d2, s.b[3], v);
+  } else {
+    s.b[0] = fma(d, s.b[0], ya);
+    s.b[1] = fma(d, s.b[1], yb);
+    s.b[2] = fma(d, s.b[2], ya * yb);
+    s.b[3] = fma(d, s.b[3], v);
+    s.b[4] = fma(d2, s.b[4], v);
+    if constexpr (KIND == kECorr) {
+      s.b[5] = fma(d, s.b[5], ya * ya);
+      s.b[6] = fma(d, s.b[6], yb * yb);
+    }
+  }
+  if constexpr (WT) s.b[Sp::NS - 1] = fma(d, s.b[Sp::NS - 1], v * alpha);
+}
+
+// a b - c d with the second product's rounding error taken off again.
+__device__ __forceinline__ double diff_prod(double a, double b, double c, double d) {
+  const double p = c * d;
+  return fma(a, b, -p) - fma(c, d, -p);
+}
+// a / b for |a| <= 2**500 and 2**-500 <= |b| <= 2**500 (div_rn).
+__device__ __forceinline__ double fast_div(double a, double b) { return div_rn(a, b, recip_refined(b)); }
+
+// Outputs. With w = sum_weight the reference's
+//   (sum_x2 / w - (sum_x / w)^2) / (1 - sum_w2 / w^2) = (sum_x2 w - sum_x^2) / (w^2 - sum_w2)
+// takes one division instead of five (cov alike; corr's weights cancel:
+// (s12 w - s1 s2) / sqrt((s11 w - s1^2)(s22 w - s2^2))), and the bias test
+// 1 - sum_w2 / w^2 > 0 is w^2 > sum_w2. Tiny weights (long gaps) and numerators
+// beyond 2**500 take the reference's own form.
+template <int KIND, bool WT>
+__device__ __forceinline__ double uni_out(const UState<UniSpec<KIND, WT>::NS>& s, double mw) {
+  using Sp = UniSpec<KIND, WT>;
+  const double nan = canonical_nan<double>();
+  const double* b = s.b;
+  const bool heavy = WT ? b[Sp::NS - 1] >= mw : true;
+  if constexpr (KIND == kECount) return heavy ? b[0] : nan;
+  if constexpr (KIND == kESum) return heavy && s.seen ? b[0] : nan;
+  if constexpr (KIND == kEMean) {
+    const double m = recip_range(b[1]) && div_range(b[0]) ? fast_div(b[0], b[1]) : b[0] / b[1];
+    return heavy ? m : nan;
+  }
+  if constexpr (Sp::MOM) {
+    constexpr int W = (KIND == kEVar || KIND == kEStd) ? 2 : 3;
+    const double w = b[W], w2 = b[W + 1];
+    const double den = fma(w, w, -w2);
+    // den = bias w^2 with bias in [2**-53, 1]: a den of 2**-380 puts w above
+    // 2**-190; without the weight (0 <= alpha <= 1) w is at most n
+    const bool ok = heavy && s.seen >= 2 && den >= 0x1p-380 && (!WT || w <= 0x1p200);
+    if constexpr (KIND == kEVar || KIND == kEStd) {
+      const double num = diff_prod(b[0], w, b[1], b[1]);
+      if (__builtin_expect(ok && div_range(num), 1)) {
+        if (KIND == kEVar) return fast_div(num, den);
+        if (num >= 0x1p-500) return num * rsqrt_refined(num * den);  // sqrt(num / den)
+      }
+      const double m = b[1] / w;
+      const double bias = 1.0 - w2 / (w * w);
+      if (!(heavy && bias > 0 && s.seen >= 2)) return nan;
+      const double v = (b[0] / w - m * m) / bias;
+      return KIND == kEStd ? sqrt(v) : v;
+    } else if constexpr (KIND == kECov) {
+      const double num = diff_prod(b[2], w, b[0], b[1]);
+      if (__builtin_expect(ok && div_range(num), 1)) return fast_div(num, den);
+      const double bias = 1.0 - w2 / (w * w);
+      const double cov = (b[2] - b[0] * b[1] / w) / w;
+      return heavy && bias > 0 && s.seen >= 2 ? cov / bias : nan;
+    } else {
+      const double v1 = diff_prod(b[5], w, b[0], b[0]), v2 = diff_prod(b[6], w, b[1], b[1]);
+      const double vv = v1 * v2;
+      if (__builtin_expect(ok && vv >= 0x1p-1000 && vv <= 0x1p1000, 1))
+        return diff_prod(b[2], w, b[0], b[1]) * rsqrt_refined(vv);
+      const double bias = 1.0 - w2 / (w * w);
+      const double cov = b[2] - b[0] * b[1] / w;
+      const double u1 = b[5] - b[0] * b[0] / w, u2 = b[6] - b[1] * b[1] / w;
+      const double uu = u1 * u2;
+      return heavy && bias > 0 && s.seen >= 2 && uu > 0 ? cov / sqrt(uu) : nan;
+    }
+  }
+  return nan;
+}
+
+constexpr int kExpGroup = kWave;
+
+// q^m for 0 <= m < 64
+__device__ __forceinline__ double pow_bits(double q, int m) {
+  double r = 1.0;
+#pragma unroll
+  for (int i = 0; i < 6; ++i) {
+    r *= (m >> i) & 1 ? q : 1.0;
+    q *= q;
+  }
+  return r;
+}
+
+// Wave: the state of `cnt` consecutive tiles (prow: the first one's payload),
+// in every lane.
+template <int NS, int SW2>
+__device__ __forceinline__ UState<NS> uni_join_tiles(const double* prow, int cnt, double ptile) {
+  const int lane = lane_id();
+  UState<NS> v;
+  const double q = pow_bits(ptile, lane < cnt ? cnt - 1 - lane : 0);
+#pragma unroll
+  for (int c = 0; c < NS; ++c)
+    v.b[c] = lane < cnt ? prow[(int64_t)lane * kPayload + c] * (c == SW2 ? q * q : q) : 0.0;
+  v.seen = lane < cnt ? (int)prow[(int64_t)lane * kPayload + NS] : 0;
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) {
+#pragma unroll
+    for (int c = 0; c < NS; ++c) v.b[c] += __shfl_xor(v.b[c], o, kWave);
+    v.seen = join_seen(v.seen, __shfl_xor(v.seen, o, kWave));
+  }
+  return v;
+}
+
+// Modes as exp_kernel's: 0 one pass with look-back, 1 tile states to the
+// payload, 2 outputs from the incoming states in the payload.
+template <typename TX, typename TA, int KIND, bool WT, int MODE>
+__global__ __launch_bounds__(kExpThreads) void exp_uni_kernel(ExpArgs A) {
+  using Sp = UniSpec<KIND, WT>;
+  constexpr int NS = Sp::NS, SW2 = Sp::SW2;
+  constexpr int K = uni_items<TX, KIND>();
+  constexpr int TILE = kExpThreads * K;
+  using St = UState<NS>;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  __shared__ St s_wave[kExpWaves];
+  __shared__ St s_in;
+  __shared__ int s_ticket;
+
+  const uint32_t v_id = MODE == 0 ? 0u : xcd_order(blockIdx.x, gridDim.x);
+  const int64_t row = MODE == 0 ? (int64_t)(blockIdx.x % (uint64_t)A.rows)
+                                : (int64_t)(v_id / (uint64_t)A.tiles_per_row);
+  const TX* ra = static_cast<const TX*>(A.xa) + row * A.ld_a;
+  const TX* rb = (Sp::NARGS == 2) ? static_cast<const TX*>(A.xb) + row * A.ld_b : nullptr;
+  TA* ro = static_cast<TA*>(A.out) + row * A.ld_out;
+  const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
+  const int64_t n = A.n;
+  TX* la = reinterpret_cast<TX*>(smem_raw);
+  TX* lb = la + pad16(TILE) + 16;
+  int64_t tile;
+  if constexpr (MODE == 0) {
+    // tickets as in exp_kernel
+    const int64_t guess = (int64_t)(blockIdx.x / (uint64_t)A.rows);
+    if (tid == 0) s_ticket = (int)atomicAdd(&A.counters[row], 1u);
+    exp_stage<TX, Sp::NARGS, TILE>(ra, rb, n, guess, la, lb);
+    __syncthreads();
+    tile = s_ticket;
+    if (tile != guess) {
+      __syncthreads();
+      exp_stage<TX, Sp::NARGS, TILE>(ra, rb, n, tile, la, lb);
+      __syncthreads();
+    }
+  } else {
+    tile = (int64_t)(v_id % (uint64_t)A.tiles_per_row);
+    exp_stage<TX, Sp::NARGS, TILE>(ra, rb, n, tile, la, lb);
+    __syncthreads();
+  }
+  const int64_t t0 = tile * TILE;
+  const bool full = t0 + TILE <= n;
+  const int e0 = tid * K;
+  const double d = A.d, d2 = A.d2;
+  const double alpha = (double)(TA)A.alpha_scalar;
+  double ka = 0.0, kb = 0.0;
+  if constexpr (Sp::MOM) {
+    ka = exp_shift(ra, n);
+    if constexpr (Sp::NARGS == 2) kb = exp_shift(rb, n);
+  }
+  const TX kta = (TX)ka, ktb = (TX)kb;  // exact: the shift is one of the values
+  auto step = [&](St& s, int j) {
+    const TX a = la[pad16(e0 + j)];
+    const TX b = (Sp::NARGS == 2) ? lb[pad16(e0 + j)] : TX(0);
+    const bool valid = (Sp::NARGS == 2) ? !(is_nan(a) || is_nan(b)) : !is_nan(a);
+    const double ya = (double)(valid ? a : kta) - ka;  // 0 where invalid
+    const double yb = (Sp::NARGS == 2) ? (double)(valid ? b : ktb) - kb : 0.0;
+    uni_step<KIND, WT>(s, valid, ya, yb, d, d2, alpha);
+  };
+
+  // 1. this thread's state from zero. Positions past the row end are NaN: they
+  //    only decay, and nothing follows them.
+  St zero;
+#pragma unroll
+  for (int c = 0; c < NS; ++c) zero.b[c] = 0.0;
+  zero.seen = 0;
+  St m = zero;
+#pragma unroll
+  for (int j = 0; j < K; ++j) step(m, j);
+  m.seen = min(2, m.seen);
+  park_inf<KIND>(m);
+
+  // 2. wave scan: within 16-lane rows the earlier range is 2^i threads long
+  //    where it exists; the broadcasts join it to the lanes' own prefixes.
+  const double p16 = ((lane & 1) ? A.pw[0] : 1.0) * ((lane & 2) ? A.pw[1] : 1.0) *
+                     (((lane & 4) ? A.pw[2] : 1.0) * ((lane & 8) ? A.pw[3] : 1.0));  // d^(K (lane % 16))
+  const double p32 = p16 * ((lane & 16) ? A.pw[4] : 1.0);
+  const double p64 = p32 * ((lane & 32) ? A.pw[5] : 1.0);
+  St incl = m;
+  incl = uni_join<NS, SW2>(uni_dpp<0x111, 0xf, NS>(incl), incl, A.pw[0]);
+  incl = uni_join<NS, SW2>(uni_dpp<0x112, 0xf, NS>(incl), incl, A.pw[1]);
+  incl = uni_join<NS, SW2>(uni_dpp<0x114, 0xf, NS>(incl), incl, A.pw[2]);
+  incl = uni_join<NS, SW2>(uni_dpp<0x118, 0xf, NS>(incl), incl, A.pw[3]);
+  incl = uni_join<NS, SW2>(uni_dpp<0x142, 0xa, NS>(incl), incl, p16 * A.pw[0]);
+  incl = uni_join<NS, SW2>(uni_dpp<0x143, 0xc, NS>(incl), incl, p32 * A.pw[0]);
+  St excl = uni_dpp<0x138, 0xf, NS>(incl);  // wave_shr:1
+  if (lane == kWave - 1) s_wave[wave] = incl;
+  if (MODE == 2 && wave == 0) {  // the group's incoming state, then the group's tiles before this one
+    const int64_t g0 = tile / kExpGroup * kExpGroup;
+    const double* pl = A.payload + (row * A.tiles_per_row + g0) * kPayload;
+    const int cnt = (int)(tile - g0);
+    const St before = uni_join_tiles<NS, SW2>(pl, cnt, A.ptile);
+    St in;
+#pragma unroll
+    for (int c = 0; c < NS; ++c) in.b[c] = pl[kMaxNS + 3 + c];
+    in.seen = (int)pl[kMaxNS + 3 + NS];
+    if (lane == 0) s_in = uni_join<NS, SW2>(in, before, pow_bits(A.ptile, cnt));
+  }
+  __syncthreads();
+  const double q64 = A.pw[6];
+  if constexpr (MODE == 1) {
+    if (tid == 0) {
+      St agg = s_wave[0];
+      for (int w = 1; w < kExpWaves; ++w) agg = uni_join<NS, SW2>(agg, s_wave[w], q64);
+      double* pl = A.payload + (row * A.tiles_per_row + tile) * kPayload;
+#pragma unroll
+      for (int c = 0; c < NS; ++c) pl[c] = agg.b[c];
+      pl[NS] = (double)agg.seen;
+    }
+    return;
+  }
+  double px = p64;  // decay from the tile's start to this thread's positions
+  {
+    St wp = zero;
+    for (int w = 0; w < wave; ++w) {
+      wp = uni_join<NS, SW2>(wp, s_wave[w], q64);
+      px *= q64;
+    }
+    excl = uni_join<NS, SW2>(wp, excl, p64);
+  }
+
+  // 3. the tile's incoming state. Look-back by wave 0: lane l reads tile
+  //    top - 63 + l; published states above the highest unpublished tile, and
+  //    above the highest inclusive state, are summed with weights
+  //    d^(TILE (63 - l)); an inclusive state enters with its lane's weight and
+  //    ends the walk.
+  if (MODE == 0 && wave == 0) {
+    unsigned int* frow = A.flags + row * A.tiles_per_row;
+    double* prow = A.payload + row * A.tiles_per_row * kPayload;
+    St agg = s_wave[0];
+#pragma unroll
+    for (int w = 1; w < kExpWaves; ++w) agg = uni_join<NS, SW2>(agg, s_wave[w], q64);
+    St in = zero;
+    if (tile > 0) {
+      if (lane == 0) {
+        double* pl = prow + tile * kPayload;
+#pragma unroll
+        for (int c = 0; c < NS; ++c) st_agent_f64(pl + c, agg.b[c]);
+        st_agent_f64(pl + NS, (double)agg.seen);
+        st_flag(&frow[tile], 1u);
+      }
+      const double wl = pow_bits(A.ptile, 63 - lane);  // d^(TILE (63 - lane))
+      double acc = 1.0;  // decay over the tiles summed so far
+      int64_t top = tile - 1;
+      unsigned int spins = 0;
+      while (true) {
+        const int64_t j = top - (kWave - 1) + lane;
+        const unsigned int f = j >= 0 ? ld_flag(&frow[j]) : 2u;
+        const unsigned long long ready = __ballot(f != 0u);
+        const unsigned long long inc = __ballot(f == 2u);
+        const int hnr = ready == ~0ull ? -1 : 63 - __clzll((long long)~ready);  // highest unpublished
+        const int hp = inc == 0ull ? -1 : 63 - __clzll((long long)inc);         // highest inclusive
+        if (hnr == kWave - 1) {  // the latest tile has not published yet
+          spin_pause();
+          if (++spins > kSpinLimit) {
+            if (lane == 0) atomicAdd(A.timeouts, 1u);
+            in = zero;  // expired wait (counted): continue from zero state
+            break;
+          }
+          continue;
+        }
+        const bool last = hp > hnr;
+        const int lo = last ? hp : hnr;
+        St v = zero;
+        if ((lane > lo || (last && lane == hp)) && j >= 0) {
+          const double* pj = prow + j * kPayload + (lane > lo ? 0 : kMaxNS + 3);
+#pragma unroll
+          for (int c = 0; c < NS; ++c) v.b[c] = ld_agent_f64(pj + c);
+          v.seen = (int)ld_agent_f64(pj + NS);
+          const double q = acc * wl;
+#pragma unroll
+          for (int c = 0; c < NS; ++c) v.b[c] *= c == SW2 ? q * q : q;
+        }
+#pragma unroll
+        for (int o = 1; o < kWave; o <<= 1) {
+#pragma unroll
+          for (int c = 0; c < NS; ++c) v.b[c] += __shfl_xor(v.b[c], o, kWave);
+          v.seen = join_seen(v.seen, __shfl_xor(v.seen, o, kWave));
+        }
+#pragma unroll
+        for (int c = 0; c < NS; ++c) in.b[c] += v.b[c];
+        in.seen = join_seen(in.seen, v.seen);
+        if (last) break;
+        acc *= read_lane(wl, hnr < 0 ? 0 : hnr) * (hnr < 0 ? A.ptile : 1.0);  // d^(TILE (63 - hnr))
+        top -= (kWave - 1) - hnr;
+      }
+    }
+    if (lane == 0) {  // publish the inclusive state
+      const St out = uni_join<NS, SW2>(in, agg, A.ptile);
+      double* pl = prow + tile * kPayload + kMaxNS + 3;
+#pragma unroll
+      for (int c = 0; c < NS; ++c) st_agent_f64(pl + c, out.b[c]);
+      st_agent_f64(pl + NS, (double)out.seen);
+      st_flag(&frow[tile], 2u);
+      s_in = in;
+    }
+  }
+  if constexpr (MODE == 0) __syncthreads();
+
+  // 4. re-run this thread's positions from its incoming state.
+  St s = uni_join<NS, SW2>(s_in, excl, px);
+  unpark_inf<KIND>(s);
+  TA res[K];
+#pragma unroll
+  for (int j = 0; j < K; ++j) {
+    step(s, j);
+    res[j] = (TA)uni_out<KIND, WT>(s, A.min_weight);
+  }
+  exp_store<TX, TA, Sp::NARGS, K>(res, ro, t0, n, full, smem_raw);
+}
+
+// Two-pass middle steps for one alpha: a wave joins 64 tiles' states into a
+// group's, then a workgroup per row turns its groups' states into incoming
+// states (each thread joins a run of groups, one scan over the threads carries
+// the runs, and each thread walks its run again). A group's slot is the second
+// half of its first tile's payload; the output pass joins the tiles of its
+// group that come before its own.
+template <int KIND, bool WT>
+__global__ __launch_bounds__(kExpThreads) void exp_uni_group_kernel(ExpArgs A, int64_t groups) {
+  using Sp = UniSpec<KIND, WT>;
+  constexpr int NS = Sp::NS;
+  const int64_t g = (int64_t)blockIdx.x * kExpWaves + wave_id();
+  if (g >= A.rows * groups) return;  // whole wave
+  const int64_t row = g / groups, t = (g % groups) * kExpGroup;
+  const int64_t left = A.tiles_per_row - t;
+  double* pl = A.payload + (row * A.tiles_per_row + t) * kPayload;
+  const UState<NS> v = uni_join_tiles<NS, Sp::SW2>(pl, (int)(left < kExpGroup ? left : kExpGroup), A.ptile);
+  if (lane_id() == 0) {
+#pragma unroll
+    for (int c = 0; c < NS; ++c) pl[kMaxNS + 3 + c] = v.b[c];
+    pl[kMaxNS + 3 + NS] = (double)v.seen;
+  }
+}
+
+constexpr int kCarryThreads = 1024;
+
+template <int KIND, bool WT>
+__global__ __launch_bounds__(kCarryThreads) void exp_uni_carry_kernel(ExpArgs A) {
+  using Sp = UniSpec<KIND, WT>;
+  constexpr int NS = Sp::NS, SW2 = Sp::SW2;
+  using St = UState<NS>;
+  __shared__ St s_wave[kCarryThreads / kWave];
+  const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
+  const int64_t T = (A.tiles_per_row + kExpGroup - 1) / kExpGroup;  // groups
+  double* prow = A.payload + (int64_t)blockIdx.x * A.tiles_per_row * kPayload + kMaxNS + 3;
+  double pg = A.ptile;  // decay over a group (the last one may hold fewer tiles; nothing follows it)
+#pragma unroll
+  for (int i = 0; i < 6; ++i) pg *= pg;
+  const int64_t run = (T + kCarryThreads - 1) / kCarryThreads;
+  const int64_t b0 = tid * run;
+  const int64_t b1 = b0 + run < T ? b0 + run : T;
+  St zero;
+#pragma unroll
+  for (int c = 0; c < NS; ++c) zero.b[c] = 0.0;
+  zero.seen = 0;
+  auto get = [&](int64_t t) {
+    St v;
+    const double* pl = prow + t * kExpGroup * kPayload;
+#pragma unroll
+    for (int c = 0; c < NS; ++c) v.b[c] = pl[c];
+    v.seen = (int)pl[NS];
+    return v;
+  };
+  St m = zero;
+  for (int64_t t = b0; t < b1; ++t) m = uni_join<NS, SW2>(m, get(t), pg);
+  // A run past the row's end holds nothing and is followed by nothing, so
+  // every run counts as `run` groups.
+  double q = 1.0;
+  for (int64_t i = 0; i < run; ++i) q *= pg;
+  double pl64 = 1.0;  // decay over the lanes before this one
+  for (int o = 1; o < kWave; o <<= 1) {
+    St e;
+#pragma unroll
+    for (int c = 0; c < NS; ++c) e.b[c] = shfl_up(m.b[c], o);
+    e.seen = shfl_up(m.seen, o);
+    if (lane >= o) m = uni_join<NS, SW2>(e, m, q);
+    if (lane & o) pl64 *= q;
+    q *= q;
+  }
+  if (lane == kWave - 1) s_wave[wave] = m;
+  __syncthreads();
+  St in;
+#pragma unroll
+  for (int c = 0; c < NS; ++c) in.b[c] = shfl_up(m.b[c], 1);
+  in.seen = shfl_up(m.seen, 1);
+  if (lane == 0) in = zero;
+  St wp = zero;
+  for (int w = 0; w < wave; ++w) wp = uni_join<NS, SW2>(wp, s_wave[w], q);
+  in = uni_join<NS, SW2>(wp, in, pl64);
+  for (int64_t t = b0; t < b1; ++t) {
+    const St v = get(t);
+    double* pl = prow + t * kExpGroup * kPayload;
+#pragma unroll
+    for (int c = 0; c < NS; ++c) pl[c] = in.b[c];
+    pl[NS] = (double)in.seen;
+    in = uni_join<NS, SW2>(in, v, pg);
   }
 }
 
@@ -755,8 +1301,8 @@ __global__ __launch_bounds__(kExpThreads) void exp_carry_kernel(ExpArgs A) {
 }
 
 template <typename TX, int KIND>
-constexpr int64_t exp_tile() {
-  return kExpThreads * (int64_t)exp_items<TX, KIND>();
+constexpr int64_t exp_tile(bool uni) {
+  return kExpThreads * (int64_t)(uni ? uni_items<TX, KIND>() : exp_items<TX, KIND>());
 }
 // The smallest tile of any kind (the workspace is sized for it).
 template <typename TX>
@@ -764,22 +1310,44 @@ constexpr int64_t exp_min_tile() {
   return kExpThreads * (64 / (int64_t)sizeof(TX));
 }
 
-// Two passes on request only (NBG_EXP_TWO_PASS=1; =0 or unset: one pass).
-// Measured on MI355X for float32 (256, 2M), alpha 0.01: with 16 positions per
-// thread sum / count took 1.99 / 2.00 ms in one pass and 1.78 / 1.75 ms in
-// two, but with 32 positions one pass takes 1.62 / 1.61 ms against 1.89 /
-// 1.85 ms in two; mean 1.77 ms in one pass, 2.12 in two; the moment kinds are
-// bound by their per-tile arithmetic, which two passes repeat (cov / corr
-// 2.73 / 3.17 ms in one pass, 3.12 / 3.38 in two).
-template <int KIND>
-bool exp_two_pass(int64_t tiles) {
-  (void)tiles;
-  return knob("NBG_EXP_TWO_PASS", 0) == 1;
+// Two passes or one. In one pass a row's tiles hand their states on 64 tiles at
+// a time, about 1.8 us each hand-over, so few rows leave the chip waiting; two
+// passes read the input twice (from the MALL where it fits) and wait for
+// nothing, at two more launches. Measured on MI355X, alpha 0.05, one against
+// two passes: float64 mean of 1 row of 10M 118 against 55 us, of 16 x 1.6M 259
+// against 127, of 48 x 533k 159 against 136; float32 corr of 16 x 1.6M 202
+// against 174, of 48 x 533k 249 against 246, of 64 x 1.25M 393 against 434;
+// with fewer than 768 tiles in all, one pass is faster by the launches
+// (float32 corr of 390 tiles 32 against 35 us). The small states of float64
+// count, mean and sum hand over the least per wait: they gain up to 96 rows
+// (mean of 64 x 625k 215 against 178 us, of 128 x 312k 171 against 180). An
+// array of alphas takes one pass. NBG_EXP_TWO_PASS=0 / 1 forces either.
+template <typename TX, int KIND>
+bool exp_two_pass(const ExpArgs& a, int64_t tiles) {
+  const long long k = knob("NBG_EXP_TWO_PASS", -1);
+  if (k == 0 || k == 1) return k == 1;
+  const int64_t most = sizeof(TX) == 8 && KIND <= kESum ? 96 : 32;
+  return a.alpha == nullptr && a.rows <= most && a.rows * tiles >= 768;
+}
+
+template <typename TX, typename TA, int KIND, bool WT>
+void exp_uni_launch(const ExpArgs& a, bool two, dim3 grid, dim3 block, size_t lds, hipStream_t s) {
+  if (two) {
+    hipLaunchKernelGGL((exp_uni_kernel<TX, TA, KIND, WT, 1>), grid, block, lds, s, a);
+    const int64_t groups = (a.tiles_per_row + kExpGroup - 1) / kExpGroup;
+    hipLaunchKernelGGL((exp_uni_group_kernel<KIND, WT>), dim3((unsigned)((a.rows * groups + kExpWaves - 1) / kExpWaves)),
+                       block, 0, s, a, groups);
+    hipLaunchKernelGGL((exp_uni_carry_kernel<KIND, WT>), dim3((unsigned)a.rows), dim3(kCarryThreads), 0, s, a);
+    hipLaunchKernelGGL((exp_uni_kernel<TX, TA, KIND, WT, 2>), grid, block, lds, s, a);
+  } else {
+    hipLaunchKernelGGL((exp_uni_kernel<TX, TA, KIND, WT, 0>), grid, block, lds, s, a);
+  }
 }
 
 template <typename TX, typename TA, int KIND>
 int exp_launch(ExpArgs a, void* ws, size_t ws_bytes, hipStream_t s) {
-  const int64_t tiles = (a.n + exp_tile<TX, KIND>() - 1) / exp_tile<TX, KIND>();
+  const int64_t tile = exp_tile<TX, KIND>(a.alpha == nullptr);
+  const int64_t tiles = (a.n + tile - 1) / tile;
   const int64_t blocks = a.rows * tiles;
   if (blocks > 0x7fffffffLL) return set_error(NBG_ERR_INVALID, "move_exp: too many tiles");
   const size_t need = nbg_move_exp_workspace_bytes(a.rows, a.n, sizeof(TX) == 4 ? NBG_F32 : NBG_F64);
@@ -795,24 +1363,34 @@ int exp_launch(ExpArgs a, void* ws, size_t ws_bytes, hipStream_t s) {
   a.timeouts = spin_counter_ptr();
   if (a.timeouts == nullptr) return set_error(NBG_ERR_HIP, "move_exp: cannot resolve device counter");
   constexpr int NARGS = ExpSpec<KIND>::NARGS;
-  const size_t lds = (size_t)(pad16(exp_tile<TX, KIND>()) + 16) * sizeof(TX) * NARGS;
-  if (exp_two_pass<KIND>(tiles)) {
-    if (a.alpha == nullptr) {
-      hipLaunchKernelGGL((exp_kernel<TX, TA, KIND, true, 1>), dim3((unsigned)blocks), dim3(kExpThreads), lds, s, a);
-      hipLaunchKernelGGL((exp_carry_kernel<KIND>), dim3((unsigned)a.rows), dim3(kExpThreads), 0, s, a);
-      hipLaunchKernelGGL((exp_kernel<TX, TA, KIND, true, 2>), dim3((unsigned)blocks), dim3(kExpThreads), lds, s, a);
-    } else {
-      hipLaunchKernelGGL((exp_kernel<TX, TA, KIND, false, 1>), dim3((unsigned)blocks), dim3(kExpThreads), lds, s, a);
-      hipLaunchKernelGGL((exp_carry_kernel<KIND>), dim3((unsigned)a.rows), dim3(kExpThreads), 0, s, a);
-      hipLaunchKernelGGL((exp_kernel<TX, TA, KIND, false, 2>), dim3((unsigned)blocks), dim3(kExpThreads), lds, s, a);
-    }
-    return check_hip(hipGetLastError(), "exp_kernel launch");
+  const size_t lds = (size_t)(pad16(tile) + 16) * sizeof(TX) * NARGS;
+  const dim3 grid((unsigned)blocks), block(kExpThreads);
+  const bool two = exp_two_pass<TX, KIND>(a, tiles);
+  if (!two) {
+    if (int rc = launch_zero(ws, zero_bytes, s)) return rc;
   }
-  if (int rc = launch_zero(ws, zero_bytes, s)) return rc;
-  if (a.alpha == nullptr)
-    hipLaunchKernelGGL((exp_kernel<TX, TA, KIND, true>), dim3((unsigned)blocks), dim3(kExpThreads), lds, s, a);
-  else
-    hipLaunchKernelGGL((exp_kernel<TX, TA, KIND, false>), dim3((unsigned)blocks), dim3(kExpThreads), lds, s, a);
+  if (a.alpha == nullptr) {
+    constexpr int K = uni_items<TX, KIND>();
+    const double alpha = (double)(TA)a.alpha_scalar;
+    a.d = 1.0 - alpha;
+    a.d2 = a.d * a.d;
+    long double q = 1.0L;  // powers rounded once each
+    for (int i = 0; i < K; ++i) q *= (long double)a.d;
+    for (int i = 0; i < 8; ++i, q *= q) a.pw[i] = (double)q;
+    a.ptile = (double)q;
+    static_assert(kExpThreads == 256, "2^8 threads per tile");
+    const bool wt = !(a.min_weight <= 0.0 && alpha >= 0.0 && alpha <= 1.0);
+    if (wt) exp_uni_launch<TX, TA, KIND, true>(a, two, grid, block, lds, s);
+    else exp_uni_launch<TX, TA, KIND, false>(a, two, grid, block, lds, s);
+    return check_hip(hipGetLastError(), "exp_uni_kernel launch");
+  }
+  if (two) {
+    hipLaunchKernelGGL((exp_kernel<TX, TA, KIND, 1>), grid, block, lds, s, a);
+    hipLaunchKernelGGL((exp_carry_kernel<KIND>), dim3((unsigned)a.rows), block, 0, s, a);
+    hipLaunchKernelGGL((exp_kernel<TX, TA, KIND, 2>), grid, block, lds, s, a);
+  } else {
+    hipLaunchKernelGGL((exp_kernel<TX, TA, KIND>), grid, block, lds, s, a);
+  }
   return check_hip(hipGetLastError(), "exp_kernel launch");
 }
 

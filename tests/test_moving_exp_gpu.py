@@ -227,3 +227,57 @@ def test_exp_alpha_modes_and_dtypes(gpu_lib):
     # big-endian input (test_moving_exp.py:312-320)
     a = rng.random((3, 500))
     assert_allclose(nb.move_exp_nanmean(a.astype(">f8"), alpha=0.25), nb.move_exp_nanmean(a, alpha=0.25))
+
+
+@pytest.mark.parametrize("two_pass", ["0", "1", ""])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("func", FUNCS1 + FUNCS2)
+def test_exp_scalar_alpha_matches_alpha_array(gpu_lib, monkeypatch, func, dtype, two_pass):
+    """One alpha for all positions (its own kernel, in one pass or two) against
+    the same alpha as an array (the general kernel): lengths around the tiles,
+    long gaps whose weights fall below 2**-200, infinities, alphas at and beyond
+    the ends of [0, 1], weight thresholds. Both stay within 1e-12 (moments 1e-9)
+    of the exact recurrence by this file's bars, so within twice that of each
+    other."""
+    import numbagg_amd as nb
+    from oracle import exact
+
+    monkeypatch.setenv("NBG_EXP_TWO_PASS", two_pass)
+    cases = [(3, 2047, 0.3, 0), (1, 2049, 0.05, 0), (2, 4096, 1.0, 0), (2, 8193, 0.0, 0), (5, 16_385, 0.01, 0.2),
+             (1, 300_001, 0.02, -1.0), (40, 5000, 0.05, 0), (2, 700, 1.5, 0)]
+    for rows, n, alpha, mw in cases:
+        x = walk_array(rows, n, seed=n, dtype=dtype, offset=5.0)
+        y = walk_array(rows, n, seed=n + 1, dtype=dtype, offset=-3.0)
+        if n > 16_000:
+            x[0, 1000:14_000] = np.nan
+            if func in FUNCS1:  # (a co-moment's infinity is signed by the data's shift)
+                x[-1, 15_000] = np.inf
+        got = getattr(nb, func)(*_args(func, x, y), alpha=alpha, min_weight=mw)
+        if n > 16_000:
+            # the exact recurrence, in which an infinity stays: where the decay of
+            # its tile underflows, the general kernel turns it into NaN
+            want = exact.move_exp(func, x, alpha, mw, y=y if func in FUNCS2 else None, loop_dtype=np.float64)
+        else:
+            want = getattr(nb, func)(*_args(func, x, y), alpha=np.full(n, alpha), min_weight=mw)
+        assert got.dtype == want.dtype == np.float64
+        tag = f"{func} {rows}x{n} alpha {alpha}"
+        assert np.array_equal(np.isnan(got), np.isnan(want)), tag
+        ok = np.isfinite(want)
+        assert np.array_equal(got[~ok], want[~ok], equal_nan=True), tag
+        if func in MOMENTS:
+            scale = float(np.nanmax(np.abs(x[np.isfinite(x)])))
+            assert_allclose(got[ok], want[ok], rtol=2e-9, atol=2e-9 * scale**2, err_msg=tag)
+        else:
+            assert_allclose(got[ok], want[ok], rtol=2e-12, atol=2e-12 * float(np.nanmax(np.abs(x[np.isfinite(x)]))),
+                            err_msg=tag)
+
+
+def test_exp_scalar_alpha_constant_rows(gpu_lib):
+    """Rows of one value have variance and deviation exactly zero."""
+    import numbagg_amd as nb
+
+    x = np.full((2, 9000), 0.1, dtype=np.float32)
+    x[0, ::5] = np.nan
+    for func in ("move_exp_nanvar", "move_exp_nanstd"):
+        got = getattr(nb, func)(x, alpha=0.1)
+        assert np.isnan(got[:, 0]).all() and (got[:, 2:] == 0).all()
