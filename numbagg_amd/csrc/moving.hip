@@ -64,11 +64,11 @@ int move_launch_k(const T* a, const T* b, T* out, int64_t rows, int64_t n, int64
   constexpr int MAXV = 16 / (int)sizeof(T);
   const int v_use = pick_vec_elem<T>(a, Tr::NARGS == 2 ? b : a, out);
   // a reciprocal table in LDS (float32): 1/c for mean (NaN below the
-  // effective min_count), 1/max(c, 1) for the moment kinds, read instead of
+  // effective min_count), 1/max(c, 1) for var, std and cov, read instead of
   // refined reciprocals per output, which also frees registers (move_var 1.26
   // -> 1.20 ms, move_std 1.41 -> 1.31, move_cov 1.92 -> 1.88 on (256, 2M),
   // window 1000)
-  constexpr bool LUT_OK = KIND != kSum && KIND < 16 && sizeof(T) == 4;
+  constexpr bool LUT_OK = KIND != kSum && KIND != kCorr && KIND < 16 && sizeof(T) == 4;
   const bool use_lut = LUT_OK && mean_uses_lut(window);
   size_t lds = (size_t)rolling_stage_bytes<T>(KP, window, tail_lds, Tr::NARGS);
   if (use_lut) lds += (size_t)(window + 1) * sizeof(double);

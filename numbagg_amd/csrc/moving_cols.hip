@@ -54,33 +54,6 @@ struct IsMoments : std::false_type {};
 template <typename T, int NM>
 struct IsMoments<MomStats<T, NM>> : std::true_type {};
 
-template <bool SUB>
-__device__ __forceinline__ void acc_prod(D& s, double a, double b) {
-  s.v = fma(SUB ? -a : a, b, s.v);
-}
-template <bool SUB>
-__device__ __forceinline__ void acc_prod(Comp<double>& s, double a, double b) {
-  if (SUB) sub_prod(s, a, b);
-  else add_prod(s, a, b);
-}
-
-// One observation added to or removed from the moments, without branches: an
-// invalid one enters as zeros.
-template <bool SUB, typename T, int NM>
-__device__ __forceinline__ void acc_moments(MomStats<T, NM>& s, bool valid, T a, T b, T ka, T kb) {
-  using St = MomStats<T, NM>;
-  const double ya = valid ? (double)a - (double)ka : 0.0;
-  s.c += SUB ? -(int)valid : (int)valid;
-  s.s1.add(SUB ? -ya : ya);
-  if (St::SQA) acc_prod<SUB>(s.s11, ya, ya);
-  if (St::B) {
-    const double yb = valid ? (double)b - (double)kb : 0.0;
-    s.s2.add(SUB ? -yb : yb);
-    acc_prod<SUB>(s.s12, ya, yb);
-    if (St::SQB) acc_prod<SUB>(s.s22, yb, yb);
-  }
-}
-
 // c * s12 - s1 * s2 (c times the co-moment about the mean) of double-double
 // sums, rounded once: the products keep their low parts, so data far from the
 // lane's shift loses nothing here.

@@ -197,6 +197,34 @@ struct MomStats {
   }
 };
 
+template <bool SUB>
+__device__ __forceinline__ void acc_prod(D& s, double a, double b) {
+  s.v = fma(SUB ? -a : a, b, s.v);
+}
+template <bool SUB>
+__device__ __forceinline__ void acc_prod(Comp<double>& s, double a, double b) {
+  if (SUB) sub_prod(s, a, b);
+  else add_prod(s, a, b);
+}
+
+// One observation added to or removed from the moments, without branches: an
+// invalid one enters as zeros.
+template <bool SUB, typename T, int NM>
+__device__ __forceinline__ void acc_moments(MomStats<T, NM>& s, bool valid, T a, T b, T ka, T kb) {
+  using St = MomStats<T, NM>;
+  // an invalid observation becomes the shift (one select of T), so zero after it
+  const double ya = (double)(valid ? a : ka) - (double)ka;
+  s.c += SUB ? -(int)valid : (int)valid;
+  s.s1.add(SUB ? -ya : ya);
+  if (St::SQA) acc_prod<SUB>(s.s11, ya, ya);
+  if (St::B) {
+    const double yb = (double)(valid ? b : kb) - (double)kb;
+    s.s2.add(SUB ? -yb : yb);
+    acc_prod<SUB>(s.s12, ya, yb);
+    if (St::SQB) acc_prod<SUB>(s.s22, yb, yb);
+  }
+}
+
 // 1/c for a positive count: hardware reciprocal plus one Newton step (about
 // 1 ULP of float64, far below the float32 rounding of the result).
 __device__ __forceinline__ double recip(int c) {
@@ -351,26 +379,25 @@ struct Traits<T, kCorr> {
   using S = MomStats<T, 2>;
   static constexpr int NARGS = 2;
   static constexpr bool SHIFT = true;
-  // float32: the correlation from r = 1/max(c, 1)
-  __device__ static T from_r(const S& s, int64_t mce, double r) {
-    const double ma = s.s1.to_double() * r, mb = s.s2.to_double() * r;
-    const double va = s.s11.to_double() * r - ma * ma;
-    const double vb = s.s22.to_double() * r - mb * mb;
-    const double cv = s.s12.to_double() * r - ma * mb;
+  // float32: from c times the (co-)moments about the means, whose factors
+  // cancel, so neither 1/c nor a table of it is needed
+  // (c s12 - s1 s2) / sqrt((c s11 - s1^2)(c s22 - s2^2))
+  __device__ static T from_sums(const S& s, int64_t mce) {
+    const double c = (double)s.c, s1 = s.s1.to_double(), s2 = s.s2.to_double();
+    const double va = fma(c, s.s11.to_double(), -(s1 * s1));
+    const double vb = fma(c, s.s22.to_double(), -(s2 * s2));
+    const double cv = fma(c, s.s12.to_double(), -(s1 * s2));
     const double vv = va * vb;
     const bool in_range = vv > 0x1p-1000 && vv < 0x1p1000;
     double res = cv * rsqrt_refined(in_range ? vv : 1.0);
     if (!in_range && vv > 0) res = cv / sqrt(vv);  // extreme scales only
     return (T)((s.c >= mce && vv > 0) ? res : canonical_nan<double>());
   }
-  // float32 with the reciprocal table (the value recip forms)
-  __device__ static T out_tab(const S& s, int64_t mc, const double* rc) {
-    return from_r(s, mc > 1 ? mc : 1, rc[s.c]);
-  }
+  __device__ static T out_tab(const S& s, int64_t mc, const double*) { return from_sums(s, mc > 1 ? mc : 1); }
   __device__ static T out(const S& s, int64_t mc, const double* = nullptr) {
     const int64_t mce = mc > 1 ? mc : 1;
     if constexpr (sizeof(T) == 4) {
-      return from_r(s, mce, recip(s.c > 0 ? s.c : 1));
+      return from_sums(s, mce);
     } else {
       if (s.c < mce) return canonical_nan<T>();
       const double r = 1.0 / (double)s.c;
@@ -746,14 +773,24 @@ __device__ __forceinline__ void rolling_tile(const T* __restrict__ ra, const T* 
       res[j] = Tr::out(st, min_count, lut);
     }
   } else {
+    // float32: branch-free, one fused multiply-add per product; the
+    // double-double sums of float64 data skip invalid observations instead
+    auto add = [&](S& s, T a, T b) {
+      if constexpr (sizeof(T) == 4) acc_moments<false>(s, valid(a, b), a, b, ka, kb);
+      else if (valid(a, b)) s.add_obs(a, b, ka, kb);
+    };
+    auto sub = [&](S& s, T a, T b) {
+      if constexpr (sizeof(T) == 4) acc_moments<true>(s, valid(a, b), a, b, ka, kb);
+      else if (valid(a, b)) s.sub_obs(a, b, ka, kb);
+    };
     S delta = S::zero();
 #pragma unroll
     for (int j = 0; j < K; ++j) {
       T a, b;
       head(j, a, b);
-      if (valid(a, b)) delta.add_obs(a, b, ka, kb);
+      add(delta, a, b);
       tail(j, a, b);
-      if (valid(a, b)) delta.sub_obs(a, b, ka, kb);
+      sub(delta, a, b);
     }
     S w0_total;
     S st = block_excl_scan_and_total(delta, w0, w0_total, sh, rs.sh_w);
@@ -764,9 +801,9 @@ __device__ __forceinline__ void rolling_tile(const T* __restrict__ ra, const T* 
     for (int j = 0; j < K; ++j) {
       T a, b;
       head(j, a, b);
-      if (valid(a, b)) st.add_obs(a, b, ka, kb);
+      add(st, a, b);
       tail(j, a, b);
-      if (valid(a, b)) st.sub_obs(a, b, ka, kb);
+      sub(st, a, b);
       if constexpr (LUT) res[j] = Tr::out_tab(st, min_count, lut);  // c in [0, window]
       else res[j] = Tr::out(st, min_count, nullptr);
     }
