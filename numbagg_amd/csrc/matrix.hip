@@ -455,6 +455,249 @@ __global__ __launch_bounds__(kMxThreads) void mx_small_kernel(MxStaticArgs a) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// Static matrices of very few variables over a large batch: a wave (or the W
+// waves of a workgroup) per batch row. Lanes take 16 bytes of consecutive
+// observations of every variable and keep all sums of the row in registers:
+// P_ij = sum y_i y_j (i <= j), S_ij = sum y_i m_j, Q_ij = sum y_i^2 m_j, with
+// y = valid ? x - shift : 0 and m = valid; the pair counts are popcounts of the
+// validity ballots on the scalar unit. One pass over the row, no LDS until the
+// end, where the sums are halved across lanes by permlane swaps (two values
+// become one register of both), added along 16-lane rows and handed to one
+// lane per output. Deterministic: every order is fixed.
+//
+// Bound by float64 arithmetic (about 90 VALU instructions per 64 observations
+// of 5 variables) beside the input read: float32 (30000, 5, 1000) corr
+// 349 us in mx_small_kernel (a workgroup per row, staged in LDS, and a pass of
+// its own for the shifts), 208 here; (512, 5, 100000) 866 -> 260 us.
+// ---------------------------------------------------------------------------
+template <bool CORR>
+constexpr int tiny_max_vars() {
+  return CORR ? 5 : 6;  // the sums fit the registers of two waves per SIMD
+}
+
+// a and b, both summed over lane pairs 32 (or 16) apart, in one register: lanes
+// with that bit clear hold a's sums, the others b's.
+__device__ __forceinline__ double swap_add32(double a, double b) {
+  const unsigned long long x = (unsigned long long)__double_as_longlong(a), y = (unsigned long long)__double_as_longlong(b);
+  const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+  return __longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0])) +
+         __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
+}
+__device__ __forceinline__ double swap_add16(double a, double b) {
+  const unsigned long long x = (unsigned long long)__double_as_longlong(a), y = (unsigned long long)__double_as_longlong(b);
+  const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+  return __longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0])) +
+         __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
+}
+// Sum over the lane's row of 16, in every lane of it (row_ror reads a lane of
+// the row for every lane, so the moves need no old value).
+template <int CTRL>
+__device__ __forceinline__ double add_dpp(double v) {
+  const long long x = __double_as_longlong(v);
+  const unsigned int lo = (unsigned int)__builtin_amdgcn_mov_dpp((int)x, CTRL, 0xf, 0xf, true);
+  const unsigned int hi = (unsigned int)__builtin_amdgcn_mov_dpp((int)(x >> 32), CTRL, 0xf, 0xf, true);
+  return v + __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+__device__ __forceinline__ double row_sum(double v) {
+  return add_dpp<0x121>(add_dpp<0x122>(add_dpp<0x124>(add_dpp<0x128>(v))));  // row_ror:8, 4, 2, 1
+}
+
+template <typename T, bool CORR, int V, int W>
+__global__ __launch_bounds__(kMxThreads) void mx_tiny_kernel(MxStaticArgs a) {
+  constexpr int VE = 16 / (int)sizeof(T);  // observations per lane and step
+  constexpr int CH = kWave * VE;
+  constexpr int NPAIR = V * (V + 1) / 2, NS = V * V, NQ = CORR ? V * V : 0;
+  constexpr int TOT = NPAIR + NS + NQ, H = (TOT + 3) / 4;  // a quarter of the sums per row of 16 lanes
+  __shared__ double s_sum[kMxWaves][4 * H];
+  __shared__ int s_cnt[kMxWaves][NPAIR];
+  const int wave = mx_wave_id(), lane = threadIdx.x & (kWave - 1);
+  const int64_t b = W == 1 ? (int64_t)blockIdx.x * kMxWaves + wave : (int64_t)blockIdx.x;
+  const bool live = b < a.batch;  // uniform per wave
+  const T* x = static_cast<const T*>(a.x) + (live ? b : 0) * V * a.nobs;
+  const int64_t n = a.nobs;
+  struct Vec {
+    T v[VE];
+  };
+  auto load = [&](Vec (&q)[V], int64_t o0) {
+    const int64_t o = o0 + lane * VE;
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+      const T* p = x + v * n + o;
+      if (o0 + CH <= n) {  // 16-byte loads at element alignment
+        q[v] = load_stream(reinterpret_cast<const Vec*>(p));
+      } else {
+#pragma unroll
+        for (int e = 0; e < VE; ++e) q[v].v[e] = o + e < n ? p[e] : mx_nan<T>();
+      }
+    }
+  };
+  double P[NPAIR], S[NS], Q[CORR ? NS : 1];
+  int cnt[NPAIR];
+  double sh[V];
+  bool inf = false;
+#pragma unroll
+  for (int k = 0; k < NPAIR; ++k) P[k] = 0.0, cnt[k] = 0;
+#pragma unroll
+  for (int k = 0; k < NS; ++k) S[k] = 0.0;
+#pragma unroll
+  for (int k = 0; k < (CORR ? NS : 1); ++k) Q[k] = 0.0;
+
+  if (live) {
+    Vec cur[V], nxt[V];
+    load(cur, 0);
+    // Shifts: a finite value of each variable from the row's first observations.
+    unsigned int missing = 0;
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+      sh[v] = 0.0;
+      bool found = false;
+#pragma unroll
+      for (int e = 0; e < VE; ++e) {
+        const unsigned long long m = __ballot(fabs((double)cur[v].v[e]) < __builtin_inf());
+        if (!found && m) {
+          sh[v] = read_lane((double)cur[v].v[e], __ffsll((long long)m) - 1);
+          found = true;
+        }
+      }
+      missing |= found ? 0u : 1u << v;
+    }
+    if (__builtin_expect(missing != 0, 0)) {
+#pragma unroll 1
+      for (int v = 0; v < V; ++v) {
+        double found = 0.0;
+        if (!(missing >> v & 1)) continue;
+        for (int64_t o = 0; o < n; o += kWave) {
+          const T val = o + lane < n ? x[v * n + o + lane] : mx_nan<T>();
+          const unsigned long long m = __ballot(fabs((double)val) < __builtin_inf());
+          if (m) {
+            found = read_lane((double)val, __ffsll((long long)m) - 1);
+            break;
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < V; ++u) sh[u] = u == v ? found : sh[u];
+      }
+    }
+    const int64_t first = W == 1 ? 0 : (int64_t)wave * CH;
+    if (W > 1 && first < n) load(cur, first);
+    for (int64_t o = first; o < n; o += (int64_t)W * CH) {
+      if (o + W * CH < n) load(nxt, o + W * CH);
+#pragma unroll
+      for (int e = 0; e < VE; ++e) {
+        double y[V], m[V];
+        unsigned long long ok[V];
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+          const T t = cur[v].v[e];
+          ok[v] = __ballot(t == t);
+          y[v] = t == t ? (double)t - sh[v] : 0.0;
+          m[v] = t == t ? 1.0 : 0.0;
+          inf = inf || fabs((double)t) == __builtin_inf();
+        }
+        int k = 0;
+#pragma unroll
+        for (int i = 0; i < V; ++i)
+#pragma unroll
+          for (int j = i; j < V; ++j) cnt[k++] += __popcll(ok[i] & ok[j]);
+        k = 0;
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+          const double q = y[i] * y[i];
+#pragma unroll
+          for (int j = 0; j < V; ++j) {
+            if (j >= i) {
+              P[k] = j == i ? P[k] + q : fma(y[i], y[j], P[k]);
+              ++k;
+            }
+            S[i * V + j] = j == i ? S[i * V + j] + y[i] : fma(y[i], m[j], S[i * V + j]);
+            if (CORR && j != i) Q[CORR ? i * V + j : 0] = fma(q, m[j], Q[CORR ? i * V + j : 0]);
+          }
+        }
+      }
+#pragma unroll
+      for (int v = 0; v < V; ++v) cur[v] = nxt[v];
+    }
+  }
+  // Sums over the lanes: a quarter of them per 16-lane row.
+  double all[4 * H];
+#pragma unroll
+  for (int k = 0; k < 4 * H; ++k)
+    all[k] = k < NPAIR ? P[k < NPAIR ? k : 0]
+             : k < NPAIR + NS ? S[k < NPAIR + NS ? k - NPAIR : 0]
+             : k < TOT ? Q[(CORR && k < TOT) ? k - NPAIR - NS : 0] : 0.0;
+  const int quarter = lane >> 4;  // rows 0..3 hold sums k, k + H, k + 2 H, k + 3 H
+#pragma unroll
+  for (int k = 0; k < H; ++k) {
+    const double v = row_sum(swap_add16(swap_add32(all[k], all[k + 2 * H]), swap_add32(all[k + H], all[k + 3 * H])));
+    if ((lane & 15) == 0) s_sum[wave][quarter * H + k] = v;
+  }
+  if (lane == 0) {
+#pragma unroll
+    for (int k = 0; k < NPAIR; ++k) s_cnt[wave][k] = cnt[k];
+  }
+  if (__builtin_expect(live && __ballot(inf) != 0ull, 0)) {
+    // An infinity times a missing value's zero was NaN: this wave's sums again,
+    // pair by pair, by selection.
+#pragma unroll 1
+    for (int ij = 0; ij < V * V; ++ij) {
+      const int i = ij / V, j = ij % V;
+      double hi = 0.0, hj = 0.0;
+#pragma unroll
+      for (int v = 0; v < V; ++v) {
+        hi = v == i ? sh[v] : hi;
+        hj = v == j ? sh[v] : hj;
+      }
+      double p = 0.0, si = 0.0, qi = 0.0;
+      for (int64_t o0 = W == 1 ? 0 : (int64_t)wave * CH; o0 < n; o0 += (int64_t)W * CH) {
+        for (int e = 0; e < VE; ++e) {
+          const int64_t o = o0 + lane * VE + e;
+          if (o >= n) continue;
+          const T ti = x[i * n + o], tj = x[j * n + o];
+          if (!(ti == ti && tj == tj)) continue;
+          const double u = (double)ti - hi;
+          p += u * ((double)tj - hj);
+          si += u;
+          qi += u * u;
+        }
+      }
+#pragma unroll
+      for (int o = 1; o < kWave; o <<= 1) {
+        p += __shfl_xor(p, o, kWave);
+        si += __shfl_xor(si, o, kWave);
+        qi += __shfl_xor(qi, o, kWave);
+      }
+      if (lane == 0) {
+        if (j >= i) s_sum[wave][i * V - i * (i - 1) / 2 + (j - i)] = p;
+        s_sum[wave][NPAIR + ij] = si;
+        if (CORR) s_sum[wave][(CORR ? NPAIR + NS : 0) + ij] = qi;
+      }
+    }
+  }
+  __syncthreads();
+  if (live && (W == 1 || wave == 0) && lane < V * V) {
+    const int i = lane / V, j = lane % V;
+    const int lo = i < j ? i : j, hi = i < j ? j : i;
+    const int pk = lo * V - lo * (lo - 1) / 2 + (hi - lo);
+    double p = 0.0, si = 0.0, sj = 0.0, qi = 0.0, qj = 0.0;
+    int c = 0;
+    for (int w = 0; w < W; ++w) {
+      const double* t = s_sum[W == 1 ? wave : w];
+      p += t[pk];
+      si += t[NPAIR + i * V + j];
+      sj += t[NPAIR + j * V + i];
+      if (CORR) {
+        qi += i == j ? t[pk] : t[NPAIR + NS + i * V + j];
+        qj += i == j ? t[pk] : t[NPAIR + NS + j * V + i];
+      }
+      c += s_cnt[W == 1 ? wave : w][pk];
+    }
+    static_cast<T*>(a.out)[b * V * V + lane] = (T)static_value<CORR>(p, si, sj, (double)c, qi, qj, i == j);
+  }
+}
+
 // Launch plan: wave tile, observation splits, workspace layout.
 struct StaticPlan {
   int tw;
@@ -909,12 +1152,48 @@ bool grids_fit(std::initializer_list<int64_t> waves) {
   return true;
 }
 
+// Batches for mx_tiny_kernel: as many rows as mx_small_kernel asks for, fewer
+// variables (the sums of more do not fit a lane's registers).
+bool mx_tiny_ok(bool corr, int64_t batch, int64_t nv) {
+  return nv <= (corr ? tiny_max_vars<true>() : tiny_max_vars<false>()) && batch >= kSmallMinBatch &&
+         batch <= 0x7fffffffLL && knob("NBG_MATRIX_SMALL", 1) != 0;
+}
+
 template <typename T>
 int static_launch(bool corr, const void* x, void* out, int64_t batch, int64_t nv, int64_t nobs, void* ws,
                   hipStream_t s) {
   const StaticPlan p = static_plan(batch, nv, nobs, corr);
   if (!grids_fit({batch * nv, batch * p.tiles * p.splits, batch * p.tiles * 64}))
     return set_error(NBG_ERR_INVALID, "matrix: batch too large for one launch");
+  if (mx_tiny_ok(corr, batch, nv)) {
+    MxStaticArgs t{x, out, nullptr, nullptr, batch, nv, nobs, 0, 0, 0, 0};
+    // one wave per row fills the chip from 8192 rows on; fewer rows of more
+    // than four steps get a workgroup each
+    const bool wide = batch < 8192 && nobs > 4 * kWave * (16 / (int64_t)sizeof(T));
+    const dim3 grid((unsigned)(wide ? batch : (batch + kMxWaves - 1) / kMxWaves)), block(kMxThreads);
+#define NBG_MX_TINY(V)                                                                             \
+  case V:                                                                                          \
+    if (corr) {                                                                                    \
+      if constexpr (V <= tiny_max_vars<true>()) {                                                  \
+        if (wide) hipLaunchKernelGGL((mx_tiny_kernel<T, true, V, kMxWaves>), grid, block, 0, s, t); \
+        else hipLaunchKernelGGL((mx_tiny_kernel<T, true, V, 1>), grid, block, 0, s, t);            \
+      }                                                                                            \
+    } else {                                                                                       \
+      if (wide) hipLaunchKernelGGL((mx_tiny_kernel<T, false, V, kMxWaves>), grid, block, 0, s, t); \
+      else hipLaunchKernelGGL((mx_tiny_kernel<T, false, V, 1>), grid, block, 0, s, t);             \
+    }                                                                                              \
+    break
+    switch (nv) {
+      NBG_MX_TINY(1);
+      NBG_MX_TINY(2);
+      NBG_MX_TINY(3);
+      NBG_MX_TINY(4);
+      NBG_MX_TINY(5);
+      NBG_MX_TINY(6);
+    }
+#undef NBG_MX_TINY
+    return check_hip(hipGetLastError(), "matrix launch");
+  }
   char* w = static_cast<char*>(ws);
   double* shift = reinterpret_cast<double*>(w);
   double* part = reinterpret_cast<double*>(w + align256(p.shift_bytes));

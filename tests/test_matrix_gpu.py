@@ -427,3 +427,39 @@ def test_matrix_edge_shapes(gpu_lib):
             _check(got, exact.matrix(f, x, alpha=0.4), f == "move_exp_nancorrmatrix", 1e-11, f"{f} {shape}",
                    _pair_counts(x))
     assert nb.move_corrmatrix(np.zeros((0, 4, 2)), window=2).shape == (0, 4, 2, 2)
+
+
+# observations around a lane's 16 bytes and a wave's step; one wave and one
+# workgroup per row (fewer than 8192 rows of many steps)
+@pytest.mark.parametrize("func", ["nancorrmatrix", "nancovmatrix"])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("nv", [1, 2, 3, 4, 5, 6])
+def test_static_few_variables_vs_exact(gpu_lib, func, dtype, nv):
+    import numbagg_amd as nb
+    from oracle import exact
+
+    for batch, nobs in ((512, 2), (515, 63), (513, 257), (600, 1030), (512, 2049), (8193, 131)):
+        x = _static_data(batch, nv, nobs, dtype, seed=nv + nobs)
+        x[1, 0] = np.nan  # a variable without a value
+        x[2, -1, : nobs // 2] = np.nan
+        _check(getattr(nb, func)(x), exact.matrix(func, x), func == "nancorrmatrix", 1e-12, f"{func} {x.shape}")
+
+
+def test_static_few_variables_infinities(gpu_lib):
+    """An infinite observation makes NaN of the pairs that hold it, not of the
+    pairs whose other variable is missing there."""
+    import numbagg_amd as nb
+    from oracle import exact
+
+    x = _static_data(512, 3, 700, np.float32, seed=1)
+    x[0, 0, 0] = x[3, 1, 650] = np.inf
+    x[0, 2, 0] = x[3, 0, 650] = np.nan
+    clean = x.copy()
+    clean[0, 0, 0] = clean[3, 1, 650] = np.nan
+    want = exact.matrix("nancovmatrix", clean)
+    got = nb.nancovmatrix(x)
+    for b, i, j in ((0, 0, 2), (3, 1, 0)):  # the pair without the infinity
+        assert abs(got[b, i, j] - want[b, i, j]) <= 1.2e-7 * abs(want[b, i, j])
+        assert np.isnan(got[b, i, i]) and got[b, i, j] == got[b, j, i]
+    assert np.isnan(got[0, 0, 1]) and np.isnan(got[3, 1, 2])
+    assert np.isfinite(got[1]).all()
