@@ -707,8 +707,18 @@ struct StaticPlan {
 
 // Waves the static kernel aims for (several per SIMD of 256 CUs).
 constexpr int64_t kStaticTargetWaves = 4096;
-// Fewest observations a split covers (keeps partials small next to the input).
-constexpr int64_t kStaticMinSpan = 4096;
+// Observations a split covers at least: kStaticSpan keeps its partial sums small
+// next to its inputs; where that leaves the chip idle, down to kStaticMinSpan
+// (eight 16-observation groups, about 5 us of a wave) up to kStaticFineWaves
+// waves. Measured on MI355X, float32, spans of at least 4096 / 512 / 256 / 128
+// to fill 4096 waves: corr of (1, 19, 4824) 166 / 41 / 26 / 18 us, of
+// (1, 22, 31545) 271 / 44 / 30 / 26, cov of (24, 25, 8131) float64
+// 216 / 56 / 46 / 43, of (2, 67, 62227) 216 / 99 / 93 / 93; but corr of
+// (268, 32, 743), 804 tiles of one span each, 59 us whole and 80 in five (the
+// splits need a kernel that adds them). Up to 1024 waves nothing is slower.
+constexpr int64_t kStaticSpan = 4096;
+constexpr int64_t kStaticFineWaves = 1024;
+constexpr int64_t kStaticMinSpan = 128;
 
 StaticPlan static_plan(int64_t batch, int64_t nv, int64_t nobs, bool corr) {
   StaticPlan p{};
@@ -720,10 +730,14 @@ StaticPlan static_plan(int64_t batch, int64_t nv, int64_t nobs, bool corr) {
   p.ntile = (nv + ts - 1) / ts;
   p.tiles = p.ntile * (p.ntile + 1) / 2;
   const int64_t items = batch * p.tiles;
-  // Whole rounds of waves: at most the target, so no last round runs a few.
-  int64_t splits = knob("NBG_MATRIX_WAVES", kStaticTargetWaves) / (items > 0 ? items : 1);
-  const int64_t max_splits = (nobs + kStaticMinSpan - 1) / kStaticMinSpan;
-  if (splits > max_splits) splits = max_splits;
+  // Whole rounds of waves: at most the target, so no last round runs a few;
+  // short spans only up to kStaticFineWaves.
+  const int64_t n = items > 0 ? items : 1;
+  int64_t splits = knob("NBG_MATRIX_WAVES", kStaticTargetWaves) / n;
+  const int64_t coarse = (nobs + kStaticSpan - 1) / kStaticSpan, fine = (nobs + kStaticMinSpan - 1) / kStaticMinSpan;
+  if (splits > coarse) splits = coarse;
+  const int64_t more = kStaticFineWaves / n < fine ? kStaticFineWaves / n : fine;
+  if (splits < more) splits = more;
   if (splits < 1) splits = 1;
   int64_t span = (nobs + splits - 1) / splits;
   span = (span + 15) / 16 * 16;
@@ -758,37 +772,49 @@ struct MoveState {
   int64_t n;
 };
 
-// Window sums of one pair: add or remove the observation (xi, xj).
+// Window sums of one pair. Observations enter and leave without branches: an
+// invalid pair becomes the shifts (two selects of T), zeros after them.
 template <typename T, bool CORR>
 struct PairSums {
   double si = 0.0, sj = 0.0, sp = 0.0, qi = 0.0, qj = 0.0;
-  int64_t n = 0;
-  __device__ __forceinline__ void add(T xi, T xj, double ci, double cj, double sign) {
-    if (xi == xi && xj == xj) {
-      const double yi = (double)xi - ci, yj = (double)xj - cj;
-      si += sign * yi;
-      sj += sign * yj;
-      sp += sign * (yi * yj);
-      if (CORR) {
-        qi += sign * (yi * yi);
-        qj += sign * (yj * yj);
-      }
-      n += sign > 0.0 ? 1 : -1;
+  int n = 0;
+  template <bool SUB>
+  __device__ __forceinline__ void add(T xi, T xj, T ti, T tj, double ci, double cj) {
+    const bool both = !__builtin_isunordered(xi, xj);
+    const double yi = (double)(both ? xi : ti) - ci, yj = (double)(both ? xj : tj) - cj;
+    si += SUB ? -yi : yi;
+    sj += SUB ? -yj : yj;
+    sp = fma(SUB ? -yi : yi, yj, sp);
+    if (CORR) {
+      qi = fma(SUB ? -yi : yi, yi, qi);
+      qj = fma(SUB ? -yj : yj, yj, qj);
     }
+    n += SUB ? -(int)both : (int)both;
   }
   // The output for the current window, in forms scaled by n so that neither
   // needs a division by n: corr = (n sp - si sj) / sqrt((n qi - si^2)(n qj -
   // sj^2)); cov = (n sp - si sj) / (n (n - 1)).
-  __device__ __forceinline__ double value(int64_t min_count, int64_t mcorr, bool diag) const {
+  __device__ __forceinline__ double value(int least, bool diag) const {
     const double dn = (double)n;
+    const double cv = fma(dn, sp, -(si * sj));
     if (CORR) {
-      if (n < mcorr) return __builtin_nan("");
-      const double vi = dn * qi - si * si, vj = dn * qj - sj * sj;
-      if (!(vi > 0.0 && vj > 0.0)) return __builtin_nan("");
-      return diag ? 1.0 : mx_corr(dn * sp - si * sj, vi * vj);
+      const double vi = fma(dn, qi, -(si * si)), vj = fma(dn, qj, -(sj * sj));
+      const double vv = vi * vj;
+      const bool ok = n >= least && vi > 0.0 && vj > 0.0;
+      const bool range = vv >= 0x1p-1000 && vv <= 0x1p1000;
+      double r = cv * mx_rsqrt(range ? vv : 1.0);
+      if (__builtin_expect(ok && !range, 0)) r = cv / sqrt(vv);
+      r = diag ? 1.0 : r;
+      return ok ? r : __builtin_nan("");
     }
-    if (n < min_count || n < 2) return __builtin_nan("");
-    return (dn * sp - si * sj) / (dn * (dn - 1.0));
+    // 1 / (n (n - 1)) by a refined reciprocal, the quotient corrected by its
+    // remainder (the rounded one but for rare ties)
+    const double den = n >= 2 ? dn * (dn - 1.0) : 2.0;
+    const double e = __builtin_amdgcn_rcp(den);
+    const double r = fma(e, fma(-den, e, 1.0), e);
+    const double q = cv * r;
+    const double res = fma(fma(-den, q, cv), r, q);
+    return n >= least ? res : __builtin_nan("");
   }
 };
 
@@ -828,26 +854,48 @@ __global__ __launch_bounds__(kMxThreads) void mx_move_kernel(MxMoveArgs a) {
   T* out = static_cast<T*>(a.out) + b * a.nobs * np;
   const double ci = a.shift[(b * a.tiles + tile) * a.nv + i];
   const double cj = a.shift[(b * a.tiles + tile) * a.nv + j];
+  const T ti = (T)ci, tj = (T)cj;  // exact: shifts are values of the data
   const bool diag = i == j;
-  const int64_t mcorr = a.min_count > 2 ? a.min_count : 2;
+  const int least = a.min_count > 2 ? (a.min_count < 0x7fffffff ? (int)a.min_count : 0x7fffffff) : 2;
   const IT step = (IT)a.nv, ostep = (IT)np, back = (IT)(a.window * a.nv);
   PairSums<T, CORR> st;
   IT oi = (IT)(t_w * a.nv + i), oj = (IT)(t_w * a.nv + j);
   int64_t t = t_w;
-  for (; t < t_start; ++t, oi += step, oj += step) st.add(x[oi], x[oj], ci, cj, 1.0);
+  for (; t < t_start; ++t, oi += step, oj += step) st.template add<false>(x[oi], x[oj], ti, tj, ci, cj);
   // Outputs (V^2 per step, most of the traffic) by streaming stores: each
   // wave writes 64 consecutive elements per step, and the lines need not stay
   // in the caches (measured on MI355X, (200000, 32) float32, window 20:
   // move_covmatrix 0.528 -> 0.448 ms, move_corrmatrix 0.60 -> 0.56 ms).
   IT oo = (IT)(t_start * np + qq);
   for (; t < t_r && t < t_end; ++t, oi += step, oj += step, oo += ostep) {
-    st.add(x[oi], x[oj], ci, cj, 1.0);
-    __builtin_nontemporal_store((T)st.value(a.min_count, mcorr, diag), &out[oo]);
+    st.template add<false>(x[oi], x[oj], ti, tj, ci, cj);
+    __builtin_nontemporal_store((T)st.value(least, diag), &out[oo]);
+  }
+  // Four steps' loads in flight; the range's last steps one by one.
+  constexpr int U = 4;
+  for (; t + U <= t_end; t += U) {
+    T hi[U], hj[U], li[U], lj[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      hi[u] = x[oi + u * step];
+      hj[u] = x[oj + u * step];
+      li[u] = x[oi + u * step - back];
+      lj[u] = x[oj + u * step - back];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      st.template add<false>(hi[u], hj[u], ti, tj, ci, cj);
+      st.template add<true>(li[u], lj[u], ti, tj, ci, cj);
+      __builtin_nontemporal_store((T)st.value(least, diag), &out[oo + u * ostep]);
+    }
+    oi += U * step;
+    oj += U * step;
+    oo += U * ostep;
   }
   for (; t < t_end; ++t, oi += step, oj += step, oo += ostep) {
-    st.add(x[oi], x[oj], ci, cj, 1.0);
-    st.add(x[oi - back], x[oj - back], ci, cj, -1.0);
-    __builtin_nontemporal_store((T)st.value(a.min_count, mcorr, diag), &out[oo]);
+    st.template add<false>(x[oi], x[oj], ti, tj, ci, cj);
+    st.template add<true>(x[oi - back], x[oj - back], ti, tj, ci, cj);
+    __builtin_nontemporal_store((T)st.value(least, diag), &out[oo]);
   }
 }
 
