@@ -49,12 +49,13 @@ __device__ __forceinline__ unsigned long long pack_carry(long long idx, float v)
   return ((unsigned long long)(idx + 1) << 32) | (unsigned long long)__float_as_uint(v);
 }
 
+// 16 bytes at element alignment, which is all that 16-byte global accesses
+// need: rows of any length and offset move 16 bytes per access (float32 ffill
+// of (1000, 400001): 614 -> 530 us).
 template <typename T>
-struct alignas(16) VecT;
-template <>
-struct alignas(16) VecT<float> { float v[4]; };
-template <>
-struct alignas(16) VecT<double> { double v[2]; };
+struct VecT {
+  T v[16 / sizeof(T)];
+};
 
 // Running "last valid value" carry: scan-order offset (or -1) plus the value.
 template <typename T>
@@ -770,8 +771,7 @@ int fill_impl_b(bool rev, const void* xv, void* ov, int64_t rows, int64_t n, int
   }
   unsigned int* to = spin_counter_ptr();
   if (to == nullptr) return set_error(NBG_ERR_HIP, "fill: cannot resolve device counter");
-  const int vx = pick_vec<T>(x, ld_x, rows), vo = pick_vec<T>(out, ld_out, rows);
-  const int vec = vx < vo ? vx : vo;
+  const int vec = pick_vec_elem<T>(x, x, out);
   constexpr int MAXV = 16 / (int)sizeof(T);
   constexpr int UV = BYTES / (int)sizeof(T) / MAXV;  // slots per thread at full vector width
   dim3 grid((unsigned)blocks), block(kFillThreads);
@@ -871,8 +871,7 @@ int fill_two_pass_impl(bool rev, const void* xv, void* ov, int64_t rows, int64_t
   FillSummary* sums = static_cast<FillSummary*>(ws);
   unsigned int* to = spin_counter_ptr();
   if (to == nullptr) return set_error(NBG_ERR_HIP, "fill: cannot resolve device counter");
-  const int vx = pick_vec<T>(x, ld_x, rows), vo = pick_vec<T>(out, ld_out, rows);
-  const int vec = vx < vo ? vx : vo;
+  const int vec = pick_vec_elem<T>(x, x, out);
   dim3 grid((unsigned)blocks), block(kFillThreads);
   // run = tiles: row-major tile order, consecutive workgroups on consecutive memory
 #define NBG_FILL_PASS1(V, U, R)                                                                          \

@@ -161,30 +161,22 @@ __device__ __forceinline__ void tile_of(int64_t t, int64_t ntile, int64_t& I, in
   J = i + t;
 }
 
-template <typename T, bool VEC>
+template <typename T>
 __device__ __forceinline__ void load4(const T* __restrict__ row, int64_t k, int64_t k_hi, bool ok, T (&v)[4]) {
-  if (VEC && ok && k + 4 <= k_hi) {
-    if constexpr (sizeof(T) == 4) {
-      const float4 f = *reinterpret_cast<const float4*>(row + k);
-      v[0] = f.x;
-      v[1] = f.y;
-      v[2] = f.z;
-      v[3] = f.w;
-    } else {
-      const double2 f0 = *reinterpret_cast<const double2*>(row + k);
-      const double2 f1 = *reinterpret_cast<const double2*>(row + k + 2);
-      v[0] = f0.x;
-      v[1] = f0.y;
-      v[2] = f1.x;
-      v[3] = f1.y;
-    }
+  if (ok && k + 4 <= k_hi) {
+    struct Quad {  // 16-byte accesses at element alignment: any row length and offset
+      T v[4];
+    };
+    const Quad q = *reinterpret_cast<const Quad*>(row + k);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = q.v[e];
   } else {
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = (ok && k + e < k_hi) ? row[k + e] : mx_nan<T>();
   }
 }
 
-template <typename T, bool CORR, int TW, bool VEC>
+template <typename T, bool CORR, int TW>
 __global__ __launch_bounds__(kMxThreads) void mx_static_kernel(MxStaticArgs a) {
   constexpr int NP = StaticSpec<CORR>::NPROD;
   constexpr int TS = 16 * TW;
@@ -226,8 +218,8 @@ __global__ __launch_bounds__(kMxThreads) void mx_static_kernel(MxStaticArgs a) {
   T vi[TW][4], vj[TW][4];
 #pragma unroll
   for (int t = 0; t < TW; ++t) {
-    load4<T, VEC>(irow[t], k_lo + 4 * q, k_hi, iok[t], vi[t]);
-    load4<T, VEC>(jrow[t], k_lo + 4 * q, k_hi, jok[t], vj[t]);
+    load4<T>(irow[t], k_lo + 4 * q, k_hi, iok[t], vi[t]);
+    load4<T>(jrow[t], k_lo + 4 * q, k_hi, jok[t], vj[t]);
   }
   for (int64_t k0 = k_lo; k0 < k_hi; k0 += 16) {
     T ni[TW][4], nj[TW][4];
@@ -235,8 +227,8 @@ __global__ __launch_bounds__(kMxThreads) void mx_static_kernel(MxStaticArgs a) {
     if (more) {
 #pragma unroll
       for (int t = 0; t < TW; ++t) {
-        load4<T, VEC>(irow[t], k0 + 16 + 4 * q, k_hi, iok[t], ni[t]);
-        load4<T, VEC>(jrow[t], k0 + 16 + 4 * q, k_hi, jok[t], nj[t]);
+        load4<T>(irow[t], k0 + 16 + 4 * q, k_hi, iok[t], ni[t]);
+        load4<T>(jrow[t], k0 + 16 + 4 * q, k_hi, jok[t], nj[t]);
       }
     }
 #pragma unroll
@@ -1257,12 +1249,10 @@ int static_launch(bool corr, const void* x, void* out, int64_t batch, int64_t nv
     else hipLaunchKernelGGL((mx_small_kernel<T, false>), dim3((unsigned)batch), dim3(kMxThreads), lds, s, a);
     return check_hip(hipGetLastError(), "matrix launch");
   }
-  const bool vec = ((uintptr_t)x % 16) == 0 && (nobs % (16 / (int64_t)sizeof(T))) == 0;
   const int grid = mx_grid(batch * p.tiles * p.splits);
 #define NBG_MX_STATIC(C, TW)                                                                                   \
   do {                                                                                                         \
-    if (vec) hipLaunchKernelGGL((mx_static_kernel<T, C, TW, true>), dim3(grid), dim3(kMxThreads), 0, s, a);   \
-    else hipLaunchKernelGGL((mx_static_kernel<T, C, TW, false>), dim3(grid), dim3(kMxThreads), 0, s, a);      \
+    hipLaunchKernelGGL((mx_static_kernel<T, C, TW>), dim3(grid), dim3(kMxThreads), 0, s, a);                   \
     if (p.splits > 1)                                                                                          \
       hipLaunchKernelGGL((mx_static_finish_kernel<T, C, TW>),                                                  \
                          dim3((unsigned)(batch * p.tiles * (256 * TW * TW / kFinishPos))), dim3(kMxThreads), 0, s,  \

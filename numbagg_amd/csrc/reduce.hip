@@ -329,7 +329,7 @@ __global__ __launch_bounds__(kRedThreads) void reduce_kernel(const T* __restrict
   Lane<T, KIND> st;
   constexpr int64_t STEP = (int64_t)kWave * VEC;
   constexpr int64_t SUPER = STEP * U;
-  struct alignas(VEC * sizeof(T)) V {
+  struct V {
     T v[VEC];
   };
   int64_t e = c0;
@@ -681,8 +681,9 @@ int reduce_impl(const T* x, TO* out, int64_t rows, int64_t n, int64_t ld, int64_
   const int64_t blocks = (items + kRedWaves - 1) / kRedWaves;
   if (blocks > 0x7fffffffLL) return set_error(NBG_ERR_INVALID, "reduce: too many rows");
   RPart* parts = static_cast<RPart*>(ws);
-  const bool vec_ok = pick_vec<T>(x, ld, rows) == VEC;
-  if (vec_ok)
+  // 16-byte loads need element alignment only: rows of any length and offset
+  // take them (float32 nanvar of (9, 32628569): 427 -> 193 us)
+  if (pick_vec_elem<T>(x, x, x) == VEC)
     hipLaunchKernelGGL((reduce_kernel<T, KIND, VEC, U>), dim3((unsigned)blocks), dim3(kRedThreads), 0, s, x, n, ld,
                        chunk, cpr, items, parts);
   else
