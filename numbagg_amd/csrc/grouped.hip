@@ -115,12 +115,14 @@ struct GArgs {
   void* out;
   int64_t rows, n, ld_v, num_labels, ddof;
   int64_t chunk, chunks_per_row;  // set per launch (launch_pass)
+  int64_t slice, slices;          // labels per workgroup of one row, and how many such slices
   // global accumulators (rows x num_labels each)
   void* acc0;
   void* acc1;
   void* acc2;           // variance finalize: counts
   void* acc3;           // kPMom: per (row, label) shift (float64 bits, NaN until set)
   const double* means;  // kPDev: per (row, label) mean
+  int sliced;           // more labels than one workgroup's LDS: slices of them (run_pass)
   int argmin;           // kPPacked / kPKey / kPKeyIdx: complement keys
   int mom;              // variance finalize: from shifted moments (kPMom) instead of two passes
 };
@@ -201,15 +203,19 @@ template <typename TV, typename TL, int PASS, bool LDS, int R, bool COUNT, int U
 __global__ __launch_bounds__(kGroupThreads) void group_pass_kernel(GArgs A) {
   using SA = typename SumAcc<TV>::type;
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  const int64_t L1 = A.num_labels;        // labels per row
+  // A slice of A.slice labels of the row, from `lo` on (R == 1 only; else all).
+  // Below, labels and slots count from lo.
+  const uint32_t v = xcd_order(blockIdx.x, gridDim.x);
+  const int64_t lo = R == 1 ? (int64_t)(v % (uint32_t)A.slices) * A.slice : 0;
+  const int64_t L1 = R == 1 && A.num_labels - lo > A.slice ? A.slice : A.num_labels - lo;  // labels per row
   const int64_t L = L1 * R;               // LDS slots (row-major: r * L1 + label)
   // Chunk-major order on XCD-consecutive logical ids: the row groups of one
   // chunk run on the same XCD back to back and read its labels from that
   // XCD's L2 after the first of them.
   const uint64_t groups = (uint64_t)((A.rows + R - 1) / R);
-  const uint32_t v = xcd_order(blockIdx.x, gridDim.x);
-  const int64_t row0 = (int64_t)(v % groups) * R;
-  const int64_t ck = (int64_t)(v / groups);
+  const uint32_t vg = R == 1 ? v / (uint32_t)A.slices : v;
+  const int64_t row0 = (int64_t)(vg % groups) * R;
+  const int64_t ck = (int64_t)(vg / groups);
   const int64_t c0 = ck * A.chunk;
   const int64_t c1 = (c0 + A.chunk < A.n) ? c0 + A.chunk : A.n;
   const int nr = (int)((A.rows - row0) < R ? (A.rows - row0) : R);  // rows present
@@ -218,11 +224,12 @@ __global__ __launch_bounds__(kGroupThreads) void group_pass_kernel(GArgs A) {
   const int tid = threadIdx.x;
 
   // Global accumulators of these rows (slot r * L1 + label, rows contiguous).
-  SA* g_s = static_cast<SA*>(A.acc0) + row0 * L1;
-  unsigned long long* g_u0 = static_cast<unsigned long long*>(A.acc0) + row0 * L1;
-  unsigned long long* g_u1 = static_cast<unsigned long long*>(A.acc1) + row0 * L1;
-  double* g_sq = static_cast<double*>(A.acc1) + row0 * L1;
-  const double* g_mean = A.means ? A.means + row0 * L1 : nullptr;
+  const int64_t g0 = row0 * A.num_labels + lo;
+  SA* g_s = static_cast<SA*>(A.acc0) + g0;
+  unsigned long long* g_u0 = static_cast<unsigned long long*>(A.acc0) + g0;
+  unsigned long long* g_u1 = static_cast<unsigned long long*>(A.acc1) + g0;
+  double* g_sq = static_cast<double*>(A.acc1) + g0;
+  const double* g_mean = A.means ? A.means + g0 : nullptr;
 
   // LDS accumulators.
   SA* l_s = reinterpret_cast<SA*>(smem_raw);
@@ -299,6 +306,7 @@ __global__ __launch_bounds__(kGroupThreads) void group_pass_kernel(GArgs A) {
   // hot_c: std::true_type on the register path for labels 0 and 1.
   auto update = [&](auto hot_c, TV v, TL lbl, int64_t i, int r) {
     constexpr bool H = decltype(hot_c)::value;
+    if constexpr (R == 1) lbl = (TL)((uint64_t)lbl - (uint64_t)lo);  // a negative label stays out of range
     if constexpr (sizeof(TL) == 4) {
       if ((uint32_t)lbl >= lim32) return;
     } else {
@@ -616,15 +624,15 @@ __global__ __launch_bounds__(kGroupThreads) void group_pass_kernel(GArgs A) {
         const unsigned int c = l_mc[l];
         if (c) {
           const double k = (double)l_mk[l];
-          unsigned long long* gk = static_cast<unsigned long long*>(A.acc3) + row0 * L1 + l;
+          unsigned long long* gk = static_cast<unsigned long long*>(A.acc3) + g0 + l;
           const unsigned long long kb = (unsigned long long)__double_as_longlong(k);
           const unsigned long long old = atomicCAS(gk, 0x7FF8000000000000ull, kb);
           const double kg = old == 0x7FF8000000000000ull ? k : __longlong_as_double((long long)old);
           const double d = k - kg;
           const double s1 = l_m1[l], s2 = l_m2[l], dc = (double)c;
-          unsafeAtomicAdd(&static_cast<double*>(A.acc0)[row0 * L1 + l], s1 + dc * d);
-          unsafeAtomicAdd(&static_cast<double*>(A.acc1)[row0 * L1 + l], s2 + 2.0 * d * s1 + dc * d * d);
-          atomicAdd(&static_cast<unsigned long long*>(A.acc2)[row0 * L1 + l], (unsigned long long)c);
+          unsafeAtomicAdd(&static_cast<double*>(A.acc0)[g0 + l], s1 + dc * d);
+          unsafeAtomicAdd(&static_cast<double*>(A.acc1)[g0 + l], s2 + 2.0 * d * s1 + dc * d * d);
+          atomicAdd(&static_cast<unsigned long long*>(A.acc2)[g0 + l], (unsigned long long)c);
         }
       }
     }
@@ -729,6 +737,19 @@ __global__ void group_finalize_kernel(GArgs A, double* means_out) {
 // LDS budget for privatised accumulators (bytes per workgroup).
 constexpr int64_t kGroupLdsBudget = 48 * 1024;
 
+// More labels than that are cut into slices, each reduced by workgroups of its
+// own that skip the other labels (the values and labels then come from the L2
+// or the MALL for all but one of them): slices of up to 78 KB, two workgroups
+// per CU, where at most kGroupMaxSlices of them cover the labels and a row has
+// eight values per label. Measured on MI355X: float32 group_nanvar of
+// (2, 68.5M), 3147 labels, 20.1 ms on global
+// atomics, 0.33 in slices; float64 group_nanargmax of (2, 37.3M), 8377
+// labels, 3.63 and 0.35 ms; float32 group_nanvar of (30, 3M), 20000 labels, 10.8
+// and 0.96 ms, group_nansum 3.59 and 0.19 ms; small calls gain too (group_nanmean
+// of (3, 40000), 4800 labels, 35 and 20 us).
+constexpr int64_t kGroupSliceBytes = 78 * 1024;
+constexpr int64_t kGroupMaxSlices = 16;
+
 // The most LDS one workgroup may use on the current device (the forced LDS
 // strategy may go up to it; the automatic choice keeps to kGroupLdsBudget).
 int64_t group_lds_max() {
@@ -789,12 +810,16 @@ int launch_pass(GArgs a, size_t lds, hipStream_t s) {
         cap > per_cu * cus)
       cap = per_cu * cus;
   }
-  const int64_t per_group = cap / groups > 1 ? cap / groups : 1;
+  if (R > 1 || !LDS || a.slices < 1) {
+    a.slice = a.num_labels;
+    a.slices = 1;
+  }
+  const int64_t per_group = cap / (groups * a.slices) > 1 ? cap / (groups * a.slices) : 1;
   int64_t chunk = (a.n + per_group - 1) / per_group;
   chunk = (chunk + 4095) / 4096 * 4096;
   a.chunk = chunk;
   a.chunks_per_row = (a.n + a.chunk - 1) / a.chunk;
-  const int64_t blocks = groups * a.chunks_per_row;
+  const int64_t blocks = groups * a.chunks_per_row * a.slices;
   if (blocks > 0x7fffffffLL) return set_error(NBG_ERR_INVALID, "group: grid too large");
   hipLaunchKernelGGL((group_pass_kernel<TV, TL, PASS, LDS, R, COUNT, U, PIPE, HOT>), dim3((unsigned)blocks),
                      dim3(kGroupThreads), LDS ? lds : 0, s, a);
@@ -855,6 +880,14 @@ int run_pass(GArgs a, bool lds, hipStream_t s) {
     return launch_rows<TV, TL, PASS, COUNT, 4>(a, (size_t)bytes(4), s);
   if (rmax >= 2 && a.rows >= 2 && bytes(2) <= kGroupLdsBudget)
     return launch_rows<TV, TL, PASS, COUNT, 2>(a, (size_t)bytes(2), s);
+  if (a.sliced && bytes(1) > kGroupLdsBudget) {
+    const int64_t most = group_lds_max() < kGroupSliceBytes ? group_lds_max() : kGroupSliceBytes;
+    a.slices = (bytes(1) + most - 1) / most;  // equal slices; a whole number of labels fits each
+    if (a.slices * (most / slot) < L) ++a.slices;
+    a.slice = (L + a.slices - 1) / a.slices;
+    a.slices = (L + a.slice - 1) / a.slice;
+    return launch_rows<TV, TL, PASS, COUNT, 1>(a, (size_t)(a.slice * slot), s);
+  }
   return launch_rows<TV, TL, PASS, COUNT, 1>(a, (size_t)bytes(1), s);
 }
 
@@ -921,6 +954,12 @@ int group_impl(GArgs a, int strategy, void* ws, size_t ws_bytes, hipStream_t s) 
     if (lds_need > group_lds_max())
       return set_error(NBG_ERR_INVALID, "group: %lld labels do not fit the LDS strategy", (long long)L);
     lds = true;
+  }
+  a.sliced = 0;
+  if (strategy == NBG_GROUP_AUTO && !lds && a.n >= 8 * L && lds_need <= kGroupMaxSlices * kGroupSliceBytes &&
+      lds_need <= kGroupMaxSlices * group_lds_max()) {
+    lds = true;
+    a.sliced = 1;
   }
   if (strategy == NBG_GROUP_GLOBAL) lds = false;
 

@@ -412,3 +412,38 @@ def test_group_rest_of_family_edge_cases(gpu_lib, func):
     empty = {"group_nanprod": 1.0, "group_nanall": 1.0, "group_nansum_of_squares": 0.0, "group_nanany": 0.0}
     got = getattr(nb, func)(np.zeros((3, 0), np.float32), np.zeros(0, np.int32), axis=-1, num_labels=2)
     np.testing.assert_array_equal(got, np.full((3, 2), empty.get(func, np.nan), np.float32))
+
+
+@pytest.mark.parametrize("ldt", [np.int32, np.int64])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("num_labels", [1760, 5001, 20_011])
+def test_label_slices(gpu_lib, monkeypatch, dtype, ldt, num_labels):
+    """More labels than one workgroup's LDS holds: slices of them (the automatic
+    choice) against the global-accumulator strategy, for every function; rows at
+    odd offsets, negative and too large labels, labels without values. Copies,
+    counts and indices are equal; float sums and moments agree within the bars
+    of this file (one float32 rounding each, or 1e-12)."""
+    import torch
+
+    import numbagg_amd as nb
+
+    rng = np.random.default_rng(num_labels)
+    n = 8 * num_labels + 1003
+    x = rng.standard_normal((3, n + 1)).astype(dtype) + 3
+    x[rng.random(x.shape) < 0.1] = np.nan
+    lab = rng.integers(-2, num_labels + 3, n).astype(ldt)
+    lab[lab == 7] = 8
+    lab[:4] = np.iinfo(ldt).min, np.iinfo(ldt).max, num_labels - 1, 0
+    t, tl = torch.from_numpy(x).cuda()[:, 1:], torch.from_numpy(lab).cuda()
+    for name in nb.grouped.__all__:
+        f = getattr(nb, name)
+        got = f(t, tl, num_labels=num_labels, axis=-1)
+        monkeypatch.setenv("NBG_GROUP_STRATEGY", "global")
+        want = f(t, tl, num_labels=num_labels, axis=-1)
+        monkeypatch.delenv("NBG_GROUP_STRATEGY")
+        g, w = got.cpu().numpy(), want.cpu().numpy()
+        assert np.array_equal(np.isnan(g), np.isnan(w)), name
+        if name.split("_nan")[1] in ("sum", "mean", "var", "std", "prod", "sum_of_squares"):
+            np.testing.assert_allclose(g, w, rtol=2.4e-7 if dtype == np.float32 else 1e-12, atol=1e-12, err_msg=name)
+        else:
+            assert np.array_equal(g, w, equal_nan=True), name
