@@ -80,3 +80,21 @@ def test_codes_drive_group_by(gpu_lib):
     t_codes, t_uniques = nb.factorize(torch.from_numpy(raw).cuda())
     assert t_codes.is_cuda and t_uniques.is_cuda
     assert_array_equal(t_codes.cpu().numpy(), codes)
+
+
+@pytest.mark.parametrize("sort", [True, False])
+@pytest.mark.parametrize(
+    ("n", "k"),
+    [(1_000, 1), (5_000, 31), (5_000, 33), (50_000, 2049), (100_000, 16_384), (100_000, 16_385),
+     (16 * 65536 - 1, 700), (16 * 65536, 700), (16 * 65536 + 1, 40_000)],
+)
+def test_ranks_and_leading_values(gpu_lib, n, k, sort):
+    """Exactly k uniques at the edges of the counted ranks (an entry per eight
+    lanes, a staged tile, the last list that is counted), and lengths around
+    the one from which the leading values go ahead: with few uniques, and with
+    more than the small table takes, found by the leading values already. The
+    uniques include the integer -1, kept outside the table."""
+    rng = np.random.default_rng(n + k)
+    v = rng.permutation(np.concatenate([np.arange(k), rng.integers(0, k, size=n - k)])) * 3 - 1
+    _check(v.astype(np.int64), sort)
+    _check(v.astype(np.float64), sort)
