@@ -18,7 +18,7 @@
 //   4. rank: each sorted entry writes its rank into its slot and its value into
 //      the uniques;
 //   5. codes: every value finds its slot again and reads the rank (for up to
-//      2048 uniques in a key -> rank table that each workgroup builds in LDS).
+//      4096 uniques in a key -> rank table that each workgroup builds in LDS).
 // The empty marker is the all-ones word: no float key can equal it (it is a
 // NaN pattern, and NaN is never inserted); the integer -1 (sign-extended to
 // the same bits) is tracked by a flag outside the table.
@@ -40,6 +40,18 @@ __device__ __forceinline__ unsigned long long mix64(unsigned long long k) {
   k *= 0xc4ceb9fe1a85ec53ull;
   k ^= k >> 33;
   return k;
+}
+
+// Hash of a key for the tables in LDS, a scaled index below `range`: three
+// 32-bit multiplications instead of the eight of mix64, which is most of the
+// arithmetic per value. Its odd constants are the leading fraction bits of the
+// golden ratio and of the square roots of two and three; keys that collide
+// only lengthen a probe.
+__device__ __forceinline__ unsigned int fz_hash(unsigned long long k, unsigned int range) {
+  unsigned int h = (unsigned int)k * 0x9E3779B1u + (unsigned int)(k >> 32) * 0x6A09E667u;
+  h ^= h >> 15;
+  h *= 0xBB67AE85u;
+  return __umulhi(h, range);
 }
 
 // The table key of a value (-0.0 folded onto +0.0) and whether it is NaN.
@@ -142,82 +154,129 @@ __device__ __forceinline__ void fz_table_insert(const FzArgs& A, const FzTable& 
 // workgroup instead of two per value. A key that finds no LDS slot within
 // kFzLdsProbe probes (the table holds kFzLdsSlots) goes to the global table
 // directly, so any number of uniques is correct.
+//
+// A launch over the first kFzLead values goes ahead of the one over all of
+// them. Every workgroup of the whole pass puts the same few keys into the
+// global table at the same time, with two atomics per key and workgroup that
+// queue at each address; with the keys and their first positions already
+// there, both checks are plain reads. Measured on MI355X, 16M int64 labels of 1000
+// uniques: with and without it, 183 and 195 us for the whole call; 50000
+// uniques, where the small table overflows at once and the pass over it ends,
+// 1363 and 1596 us; 200 uniques of 30M float64, where there is little to save,
+// 200 and 186 us. Below kFzLeadFrom values the whole pass has few workgroups
+// and the launch costs more than it saves.
+constexpr int64_t kFzLead = 65536;
+constexpr int64_t kFzLeadFrom = 16 * kFzLead;
+constexpr int64_t kFzLeadChunk = 4096;
+
+// The LDS table is probed in pairs of slots, 16 bytes of keys and 8 of first
+// positions (relative to the chunk): the home pairs of a thread's kFzUnroll
+// values are read together, and only a key outside its home pair takes the
+// probe loop. Slot by slot, some lane of 64 needed a third or fourth probe for
+// nearly every value, each a chain of an LDS read, a 64-bit comparison and a
+// branch. 72 KiB of table, two workgroups per CU, hold the keys of 4600 uniques
+// where 64 KiB with 64-bit positions held 3000. Measured on MI355X, 16M int64
+// labels, the whole call with slots and with pairs (and the leading values
+// above): 300 uniques 143 and 125 us, 1000 uniques 181 and 183 us, 3000 uniques
+// 450 and 306 us, 50000 uniques 1578 and 1363 us.
 constexpr int kFzInsThreads = 1024;
-constexpr int kFzLdsSlots = 4096;  // 64 KiB of keys and first positions
-constexpr int kFzLdsProbe = 16;
+constexpr int kFzLdsSlots = 6144;
+constexpr int kFzLdsPairs = kFzLdsSlots / 2;
+constexpr int kFzLdsProbe = 8;  // pairs
+constexpr int kFzUnroll = 4;
 
 // BIG: the second pass, into the big table, run only when the small table
 // overflowed.
 template <typename T, bool BIG>
 __global__ __launch_bounds__(kFzInsThreads) void fz_insert_kernel(const T* __restrict__ x, FzArgs A, int64_t chunk) {
-  __shared__ unsigned long long lk[kFzLdsSlots], lf[kFzLdsSlots];
-  __shared__ unsigned int lused, over;
+  __shared__ __attribute__((aligned(16))) unsigned long long lk[kFzLdsSlots];
+  __shared__ __attribute__((aligned(8))) unsigned int lf[kFzLdsSlots];
+  __shared__ unsigned int lused, over, minus_one;
   if (BIG && !A.count[3]) return;
   const FzTable t = BIG ? A.big : A.small;
   for (int j = threadIdx.x; j < kFzLdsSlots; j += kFzInsThreads) {
     lk[j] = kEmpty;
-    lf[j] = kEmpty;
+    lf[j] = ~0u;
   }
   if (threadIdx.x == 0) {
     lused = 0u;
-    over = 0u;
+    minus_one = ~0u;
+    // the leading values may have overflowed the small table already
+    over = BIG ? 0u : __atomic_load_n(&A.count[3], __ATOMIC_RELAXED);
   }
   __syncthreads();
   const int64_t lo = (int64_t)blockIdx.x * chunk;
-  const int64_t hi = lo + chunk < A.n ? lo + chunk : A.n;
-  // four values per thread in flight: their loads are issued before the
-  // first one is looked up
-  constexpr int U = 4;
-  for (int64_t i0 = lo + threadIdx.x; i0 < hi; i0 += U * kFzInsThreads) {
+  const unsigned int len = (unsigned int)(lo + chunk < A.n ? chunk : A.n - lo);  // the host keeps chunks below 2^31
+  constexpr int U = kFzUnroll;
+  for (unsigned int i0 = threadIdx.x; i0 < len; i0 += U * kFzInsThreads) {
     // once the small table has overflowed its contents are dropped: stop
     if (!BIG && __atomic_load_n(&over, __ATOMIC_RELAXED)) break;
     // a table three-quarters full (many distinct keys in this chunk) only
-    // looks keys up near their home slot and claims no more slots
+    // looks keys up near their home pair and claims no more slots
     const bool claim = __atomic_load_n(&lused, __ATOMIC_RELAXED) < (unsigned int)(kFzLdsSlots * 3 / 4);
-    const int lim = claim ? kFzLdsProbe : 4;
+    const int lim = claim ? kFzLdsProbe : 2;
     T v[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int64_t i = i0 + (int64_t)u * kFzInsThreads;
-      v[u] = i < hi ? x[i] : T(0);
+      const unsigned int i = i0 + u * kFzInsThreads;
+      v[u] = i < len ? x[lo + i] : T(0);
+    }
+    unsigned long long key[U];
+    unsigned int home[U];
+    bool nan[U];
+    ulonglong2 kk[U];
+    uint2 ff[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      key[u] = fz_key(v[u], nan[u]);
+      home[u] = fz_hash(key[u], kFzLdsPairs);
+      kk[u] = *reinterpret_cast<const ulonglong2*>(&lk[2 * home[u]]);
+      ff[u] = *reinterpret_cast<const uint2*>(&lf[2 * home[u]]);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int64_t i = i0 + (int64_t)u * kFzInsThreads;
-      if (i >= hi) continue;
-      bool nan;
-      const unsigned long long k = fz_key(v[u], nan);
-      if (nan) continue;
+      const unsigned int i = i0 + u * kFzInsThreads;
+      const unsigned long long k = key[u];
+      if (i >= len || nan[u]) continue;
       if (k == kEmpty) {  // int64 -1: outside the table
-        atomicOr(&A.count[1], 1u);
-        atomicMin(A.minus_one_first, (unsigned long long)i);
+        if (i < __atomic_load_n(&minus_one, __ATOMIC_RELAXED)) atomicMin(&minus_one, i);
         continue;
       }
-      unsigned int h = (unsigned int)mix64(k) & (kFzLdsSlots - 1);
+      if (kk[u].x == k || kk[u].y == k) {
+        if (i < (kk[u].x == k ? ff[u].x : ff[u].y)) atomicMin(&lf[2 * home[u] + (kk[u].x == k ? 0 : 1)], i);
+        continue;
+      }
+      unsigned int h = 2 * home[u];
       bool placed = false;
-      for (int p = 0; p < lim; ++p) {
-        unsigned long long cur = lk[h];
+      for (int p = 0; p < 2 * lim; ++p) {
+        unsigned long long cur = __atomic_load_n(&lk[h], __ATOMIC_RELAXED);
         if (cur == kEmpty) {
           if (!claim) break;
           cur = atomicCAS(&lk[h], kEmpty, k);
           if (cur == kEmpty) atomicAdd(&lused, 1u);
         }
         if (cur == kEmpty || cur == k) {
-          if ((unsigned long long)i < lf[h]) atomicMin(&lf[h], (unsigned long long)i);
+          atomicMin(&lf[h], i);
           placed = true;
           break;
         }
-        h = (h + 1) & (kFzLdsSlots - 1);
+        h = h + 1 == kFzLdsSlots ? 0 : h + 1;
       }
-      if (!placed) fz_table_insert<BIG>(A, t, k, (unsigned long long)i, &over);
+      if (!placed) fz_table_insert<BIG>(A, t, k, (unsigned long long)(lo + i), &over);
     }
   }
   __syncthreads();
-  if (threadIdx.x == 0 && !BIG && __atomic_load_n(&A.count[3], __ATOMIC_RELAXED)) over = 1u;
+  if (threadIdx.x == 0) {
+    if (!BIG && __atomic_load_n(&A.count[3], __ATOMIC_RELAXED)) over = 1u;
+    if (minus_one != ~0u) {
+      atomicOr(&A.count[1], 1u);
+      atomicMin(A.minus_one_first, (unsigned long long)(lo + minus_one));
+    }
+  }
   __syncthreads();
   if (over) return;
   for (int j = threadIdx.x; j < kFzLdsSlots; j += kFzInsThreads)
-    if (lk[j] != kEmpty) fz_table_insert<BIG>(A, t, lk[j], lf[j], &over);
+    if (lk[j] != kEmpty) fz_table_insert<BIG>(A, t, lk[j], (unsigned long long)(lo + lf[j]), &over);
 }
 
 // Occupied slots append (sort key, slot) to the list; the bitonic sort fixes
@@ -505,18 +564,20 @@ __global__ __launch_bounds__(kFzThreads) void fz_codes_kernel(const T* __restric
 }
 
 // Codes for at most kFzLdsCodes uniques: each workgroup builds an LDS hash
-// table (key -> rank, twice as many slots as uniques) from the ranked list,
-// then looks every value up there instead of in the global table.
-constexpr int kFzLdsCodes = 2048;
-constexpr int kFzCodeSlots = 2 * kFzLdsCodes;
+// table (key -> rank) from the ranked list, then looks every value up there
+// instead of in the global table. Pairs of slots, as in the insert pass; at
+// most two thirds of the slots are used, so every probe ends.
+constexpr int kFzCodeSlots = 6144;
+constexpr int kFzCodePairs = kFzCodeSlots / 2;
+constexpr int kFzLdsCodes = 4096;
 constexpr int kFzCodeThreads = 1024;
 
 template <typename T>
 __global__ __launch_bounds__(kFzCodeThreads) void fz_codes_lds_kernel(const T* __restrict__ x, FzArgs A,
                                                                      const long long* __restrict__ minus_one_rank,
                                                                      long long* __restrict__ codes, int64_t k_total) {
-  __shared__ unsigned long long tk[kFzCodeSlots];
-  __shared__ int tr[kFzCodeSlots];
+  __shared__ __attribute__((aligned(16))) unsigned long long tk[kFzCodeSlots];
+  __shared__ __attribute__((aligned(8))) int tr[kFzCodeSlots];
   if (fz_total(A) != k_total || k_total > kFzLdsCodes) return;
   const FzTable t = fz_table(A);
   for (int j = threadIdx.x; j < kFzCodeSlots; j += kFzCodeThreads) tk[j] = kEmpty;
@@ -524,8 +585,7 @@ __global__ __launch_bounds__(kFzCodeThreads) void fz_codes_lds_kernel(const T* _
   const int listed = (int)A.count[0];  // every unique but an int64 -1, in any order
   for (int e = threadIdx.x; e < listed; e += kFzCodeThreads) {
     const unsigned long long s = A.sval[e], k = t.keys[s];
-    // distinct keys, at most half the slots: a free slot is always found
-    for (unsigned int h = (unsigned int)mix64(k) & (kFzCodeSlots - 1);; h = (h + 1) & (kFzCodeSlots - 1)) {
+    for (unsigned int h = 2 * fz_hash(k, kFzCodePairs);; h = h + 1 == kFzCodeSlots ? 0 : h + 1) {
       if (atomicCAS(&tk[h], kEmpty, k) == kEmpty) {
         tr[h] = (int)t.rank[s];
         break;
@@ -534,18 +594,38 @@ __global__ __launch_bounds__(kFzCodeThreads) void fz_codes_lds_kernel(const T* _
   }
   __syncthreads();
   const long long m1 = *minus_one_rank;
-  for (int64_t i = (int64_t)blockIdx.x * kFzCodeThreads + threadIdx.x; i < A.n;
-       i += (int64_t)gridDim.x * kFzCodeThreads) {
-    bool nan;
-    const unsigned long long k = fz_key(x[i], nan);
-    long long c = -1;
-    if (!nan) {
-      if (k == kEmpty) {
+  constexpr int U = kFzUnroll;
+  const int64_t step = (int64_t)gridDim.x * kFzCodeThreads;
+  for (int64_t i0 = (int64_t)blockIdx.x * kFzCodeThreads + threadIdx.x; i0 < A.n; i0 += U * step) {
+    T v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = i0 + u * step < A.n ? x[i0 + u * step] : T(0);
+    unsigned long long key[U];
+    unsigned int home[U];
+    bool nan[U];
+    ulonglong2 kk[U];
+    int2 rr[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      key[u] = fz_key(v[u], nan[u]);
+      home[u] = fz_hash(key[u], kFzCodePairs);
+      kk[u] = *reinterpret_cast<const ulonglong2*>(&tk[2 * home[u]]);
+      rr[u] = *reinterpret_cast<const int2*>(&tr[2 * home[u]]);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (i0 + u * step >= A.n) break;
+      const unsigned long long k = key[u];
+      long long c = -1;
+      if (nan[u]) {
+      } else if (k == kEmpty) {
         c = m1;
+      } else if (kk[u].x == k || kk[u].y == k) {
+        c = kk[u].x == k ? rr[u].x : rr[u].y;
       } else {
         // ends at the key or at a free slot (a key not inserted: values
         // changed since the count)
-        for (unsigned int h = (unsigned int)mix64(k) & (kFzCodeSlots - 1);; h = (h + 1) & (kFzCodeSlots - 1)) {
+        for (unsigned int h = 2 * home[u];; h = h + 1 == kFzCodeSlots ? 0 : h + 1) {
           const unsigned long long ks = tk[h];
           if (ks == k) {
             c = tr[h];
@@ -554,8 +634,8 @@ __global__ __launch_bounds__(kFzCodeThreads) void fz_codes_lds_kernel(const T* _
           if (ks == kEmpty) break;
         }
       }
+      codes[i0 + u * step] = c;
     }
-    codes[i] = c;
   }
 }
 
@@ -675,18 +755,24 @@ int nbg_factorize_count(int dtype, const void* values, int64_t n, int sort, void
   const int64_t size = (int64_t)a.big.mask + 1;
   const int64_t small = (int64_t)a.small.mask + 1;
   hipLaunchKernelGGL(nbg::fz_init_kernel<false>, dim3(nbg::fz_grid(small)), dim3(nbg::kFzThreads), 0, s, a);
-  // Insert: at most 512 workgroups (two per CU in 64 KiB of LDS each), each
+  // Insert: at most 512 workgroups (two per CU in 72 KiB of LDS each), each
   // over a contiguous chunk, a multiple of the workgroup size.
   int64_t ins_blocks = (n + 16 * nbg::kFzInsThreads - 1) / (16 * nbg::kFzInsThreads);
   ins_blocks = ins_blocks < 1 ? 1 : (ins_blocks > 512 ? 512 : ins_blocks);
+  if (ins_blocks < (n >> 30)) ins_blocks = n >> 30;  // positions within a chunk are 32-bit
   int64_t chunk = (n + ins_blocks - 1) / ins_blocks;
   chunk = (chunk + nbg::kFzInsThreads - 1) / nbg::kFzInsThreads * nbg::kFzInsThreads;
   if (chunk < nbg::kFzInsThreads) chunk = nbg::kFzInsThreads;
   ins_blocks = (n + chunk - 1) / chunk;
   if (ins_blocks < 1) ins_blocks = 1;
+  nbg::FzArgs lead = a;
+  lead.n = n >= nbg::kFzLeadFrom ? nbg::kFzLead : 0;
   // small table, then (only if it overflowed: the kernels exit at once
   // otherwise) the big one
 #define NBG_FZ1(T)                                                                                          \
+  if (lead.n > 0)                                                                                            \
+    hipLaunchKernelGGL((nbg::fz_insert_kernel<T, false>), dim3((unsigned)(lead.n / nbg::kFzLeadChunk)),       \
+                       dim3(nbg::kFzInsThreads), 0, s, (const T*)values, lead, nbg::kFzLeadChunk);            \
   hipLaunchKernelGGL((nbg::fz_insert_kernel<T, false>), dim3((unsigned)ins_blocks), dim3(nbg::kFzInsThreads), \
                      0, s, (const T*)values, a, chunk);                                                     \
   hipLaunchKernelGGL(nbg::fz_init_kernel<true>, dim3(nbg::fz_grid(size)), dim3(nbg::kFzThreads), 0, s, a);    \
