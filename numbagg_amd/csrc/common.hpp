@@ -280,18 +280,6 @@ __device__ __forceinline__ void store_stream16(T* p, const T (&v)[16 / sizeof(T)
 __global__ void zero_words_kernel(unsigned long long* p, int64_t nwords);
 int launch_zero(void* p, size_t bytes, hipStream_t s);
 
-// Widest vector (in elements, up to 16 bytes) that every row of a (rows, ld)
-// view can be loaded with: the base must be aligned, and for more than one row
-// so must the row stride.
-template <typename T>
-inline int pick_vec(const void* p, int64_t ld, int64_t rows) {
-  constexpr int maxv = 16 / (int)sizeof(T);
-  for (int v = maxv; v > 1; v >>= 1) {
-    if (((uintptr_t)p % (v * sizeof(T))) == 0 && (rows <= 1 || (ld % v) == 0)) return v;
-  }
-  return 1;
-}
-
 // Widest vector for the rolling kernels, whose 16-byte global accesses need
 // element alignment only (see Vec16): MAXV elements when every pointer is
 // element-aligned, else 1.

@@ -393,7 +393,6 @@ struct Traits<T, kCorr> {
     if (!in_range && vv > 0) res = cv / sqrt(vv);  // extreme scales only
     return (T)((s.c >= mce && vv > 0) ? res : canonical_nan<double>());
   }
-  __device__ static T out_tab(const S& s, int64_t mc, const double*) { return from_sums(s, mc > 1 ? mc : 1); }
   __device__ static T out(const S& s, int64_t mc, const double* = nullptr) {
     const int64_t mce = mc > 1 ? mc : 1;
     if constexpr (sizeof(T) == 4) {
