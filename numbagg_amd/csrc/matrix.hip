@@ -38,6 +38,7 @@
 // at a chunk's start = decay product of the previous chunk x state at its
 // start + its local state), and a third replays each chunk from its carried
 // state and writes the outputs. Shifts are per variable over the whole series.
+#include <cmath>
 #include <initializer_list>
 #include <type_traits>
 
@@ -1182,6 +1183,14 @@ ExpPlan exp_plan(int64_t batch, int64_t nobs, int64_t nv, bool corr) {
   // walked one chunk after another.
   int64_t max_chunks = nobs / 64;
   if (max_chunks > kWave * 64) max_chunks = kWave * 64;
+  // And no more than balances the two: on MI355X a chunk's steps (both
+  // passes) take about 0.35 us each where few waves run, and the walk of the
+  // carry scan 0.038 us per chunk of the row, so the sum is least at sqrt(9
+  // nobs) chunks. Measured, move_exp_nancorrmatrix float32 of 300000 steps, 64
+  // chunks per lane and so: 3 variables 216 and
+  // 138 us, 5 222 and 137, 7 270 and 159, 13 356 and 318.
+  const int64_t balanced = (int64_t)std::sqrt(9.0 * (double)nobs);
+  if (max_chunks > balanced) max_chunks = balanced;
   if (max_chunks < 1) max_chunks = 1;
   if (chunks > max_chunks) chunks = max_chunks;
   if (chunks < 1) chunks = 1;

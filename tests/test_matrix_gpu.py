@@ -316,6 +316,21 @@ def test_exp_vs_exact(gpu_lib, func, dtype, case):
     _check(got, want, func == "move_exp_nancorrmatrix", 1e-11, f"{func} {case} {dtype.__name__}", _pair_counts(x))
 
 
+@pytest.mark.parametrize(("batch", "nobs", "nv"), [(1, 36_863, 3), (1, 36_865, 3), (1, 50_001, 2), (3, 50_001, 5)])
+@pytest.mark.parametrize("func", ["move_exp_nancorrmatrix", "move_exp_nancovmatrix"])
+def test_exp_balanced_chunks(gpu_lib, func, batch, nobs, nv):
+    """Around 64^2 * 9 steps, from where the number of chunks is sqrt(9 steps)
+    and no longer a chunk per 64 steps, with a last chunk of a few steps."""
+    import numbagg_amd as nb
+    from oracle import exact
+
+    x = _walk(batch, nobs, nv, np.float64, seed=nobs, offset=100.0)
+    got = getattr(nb, func)(x, alpha=0.1)
+    want = exact.matrix(func, x, alpha=0.1, loop_dtype=np.float64)
+    _check(got, want, func == "move_exp_nancorrmatrix", 1e-11, f"{func} {nobs} {nv}", _pair_counts(x))
+
+
+
 @pytest.mark.parametrize("alpha", [0.5, 0.1])
 @pytest.mark.parametrize("func", ["move_exp_nancorrmatrix", "move_exp_nancovmatrix"])
 def test_exp_pandas_goldens(gpu_lib, golden, func, alpha):
