@@ -94,11 +94,14 @@ struct FzTable {
 constexpr int64_t kFzSmallSlots = 65536;
 constexpr int kFzSmallProbe = 64;
 
+constexpr int kFzCounters = 6;  // an even number: 8-byte words follow them
+
 struct FzArgs {
   int64_t n;
   FzTable big, small;
   unsigned int* count;                 // [0] uniques in the table, [1] minus-one flag,
-                                       // [2] small-table slots taken, [3] small table overflowed
+                                       // [2] small-table slots taken, [3] small table overflowed,
+                                       // [4] compaction workgroups done
   unsigned long long* minus_one_first; // first position of an int64 -1
   unsigned long long* skey;            // sort keys (padded list)
   unsigned long long* sval;            // slot of each list entry (kEmpty: the int64 -1)
@@ -283,9 +286,10 @@ __global__ __launch_bounds__(kFzInsThreads) void fz_insert_kernel(const T* __res
 // the order. Each workgroup takes a contiguous range of slots, counts its
 // occupied ones, claims their list positions with one atomic, then writes
 // them in slot order (one atomic per workgroup: the same-address atomics of
-// per-wave claims serialise in L2, 1.5 ms for 4M uniques).
+// per-wave claims serialise in L2, 1.5 ms for 4M uniques). The last workgroup
+// with slots to claim its positions writes the number of uniques.
 template <typename T>
-__global__ __launch_bounds__(kFzThreads) void fz_compact_kernel(FzArgs A, int by_value) {
+__global__ __launch_bounds__(kFzThreads) void fz_compact_kernel(FzArgs A, int by_value, long long* uniques) {
   __shared__ unsigned int wcount[kFzThreads / 64], red[kFzThreads / 64];
   __shared__ unsigned int base;
   const FzTable t = fz_table(A);
@@ -293,6 +297,7 @@ __global__ __launch_bounds__(kFzThreads) void fz_compact_kernel(FzArgs A, int by
   int64_t per = (size + gridDim.x - 1) / gridDim.x;
   per = (per + kFzThreads - 1) / kFzThreads * kFzThreads;
   const int64_t r0 = (int64_t)blockIdx.x * per;
+  if (r0 >= size) return;  // the whole workgroup
   const int64_t r1 = r0 + per < size ? r0 + per : size;
   const int lane = __lane_id(), wave = threadIdx.x / 64;
   unsigned int c = 0u;
@@ -304,6 +309,9 @@ __global__ __launch_bounds__(kFzThreads) void fz_compact_kernel(FzArgs A, int by
     unsigned int total = 0u;
     for (int w = 0; w < kFzThreads / 64; ++w) total += red[w];
     base = total ? atomicAdd(&A.count[0], total) : 0u;
+    __threadfence();  // this claim before this workgroup's mark
+    if (atomicAdd(&A.count[4], 1u) == (unsigned int)((size + per - 1) / per) - 1u)
+      *uniques = (long long)atomicAdd(&A.count[0], 0u) + (A.count[1] ? 1 : 0);
   }
   __syncthreads();
   unsigned int off = base;
@@ -334,8 +342,6 @@ __global__ __launch_bounds__(kFzThreads) void fz_compact_kernel(FzArgs A, int by
 __device__ __forceinline__ int64_t fz_total(const FzArgs& A) {
   return (int64_t)A.count[0] + (A.count[1] ? 1 : 0);
 }
-
-__global__ void fz_total_kernel(FzArgs A, long long* total) { *total = fz_total(A); }
 
 // Entry K - 1 for an int64 -1 (value kEmpty, outside the table), and the
 // padding [K, padded): the largest key with a value above every slot, so
@@ -651,7 +657,7 @@ __global__ void fz_init_kernel(FzArgs A) {
     t.first[s] = kEmpty;
   }
   if (!BIG && blockIdx.x == 0 && threadIdx.x == 0) {
-    for (int c = 0; c < 4; ++c) A.count[c] = 0u;
+    for (int c = 0; c < kFzCounters; ++c) A.count[c] = 0u;
     *A.minus_one_first = kEmpty;
   }
 }
@@ -674,12 +680,12 @@ int64_t fz_small_size(int64_t n) {
 size_t fz_ws_bytes(int64_t n) {
   const int64_t size = fz_table_size(n) + fz_small_size(n);
   const int64_t padded = next_pow2(n + 1);
-  return (size_t)size * 24 + (size_t)padded * 16 + 32;
+  return (size_t)size * 24 + (size_t)padded * 16 + kFzCounters * 4 + 16;
 }
 
 // Workspace: keys | first | rank of the big table, then of the small one
 // (table size each, 8 bytes) | sort keys | sort values (n + 1 rounded up to
-// a power of two each) | four 32-bit counters | minus-one first position |
+// a power of two each) | kFzCounters 32-bit counters | minus-one first position |
 // minus-one rank.
 FzTable fz_table_at(char*& p, int64_t size) {
   FzTable t;
@@ -701,7 +707,7 @@ FzArgs fz_layout(int64_t n, void* ws) {
   a.skey = reinterpret_cast<unsigned long long*>(p);
   a.sval = a.skey + padded_max;
   a.count = reinterpret_cast<unsigned int*>(a.sval + padded_max);
-  a.minus_one_first = reinterpret_cast<unsigned long long*>(a.count + 4);
+  a.minus_one_first = reinterpret_cast<unsigned long long*>(a.count + kFzCounters);
   a.padded = padded_max;
   return a;
 }
@@ -779,7 +785,7 @@ int nbg_factorize_count(int dtype, const void* values, int64_t n, int sort, void
   hipLaunchKernelGGL((nbg::fz_insert_kernel<T, true>), dim3((unsigned)ins_blocks), dim3(nbg::kFzInsThreads),  \
                      0, s, (const T*)values, a, chunk);                                                     \
   hipLaunchKernelGGL((nbg::fz_compact_kernel<T>), dim3(nbg::fz_grid(size)), dim3(nbg::kFzThreads), 0, s, a,   \
-                     sort ? 1 : 0)
+                     sort ? 1 : 0, (long long*)num_uniques)
   switch (dtype) {
     case NBG_F32: NBG_FZ1(float); break;
     case NBG_F64: NBG_FZ1(double); break;
@@ -788,7 +794,6 @@ int nbg_factorize_count(int dtype, const void* values, int64_t n, int sort, void
     default: return nbg::set_error(NBG_ERR_INVALID, "nbg_factorize_count: unsupported dtype code %d", dtype);
   }
 #undef NBG_FZ1
-  hipLaunchKernelGGL(nbg::fz_total_kernel, dim3(1), dim3(1), 0, s, a, (long long*)num_uniques);
   return nbg::check_hip(hipGetLastError(), "factorize launch");
 }
 

@@ -42,7 +42,7 @@ def factorize(values, sort: bool = True):
     code = dev.nbg_code(t)
     ws_bytes = _lib.query("nbg_factorize_workspace_bytes", n)
     ws, ws_bytes = dev.workspace(ws_bytes, t.device)
-    total = torch.zeros(1, dtype=torch.int64, device=t.device)
+    total = torch.empty(1, dtype=torch.int64, device=t.device)
     stream = dev.stream_handle()
     _lib.call("nbg_factorize_count", code, dev.ptr(t), n, int(sort), dev.ptr(ws),
               ws_bytes, dev.ptr(total), stream)
