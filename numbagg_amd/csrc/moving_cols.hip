@@ -129,9 +129,10 @@ __global__ __launch_bounds__(kWave) void move_cols_kernel(MoveColsArgs A) {
   };
 
   S st = S::zero();
-  // Shift of the moment kinds: the lane's first valid value (pair) of the
-  // window before the range or of the range itself; the state is zero until
-  // then, so it can still be chosen.
+  // Shift of the moment kinds: the lane's first finite value (pair) of the
+  // window before the range or of the range itself. The state is zero until
+  // then, or holds an infinity, after which the window is summed anew, with a
+  // shift of its own.
   T ka = T(0), kb = T(0);
   bool shifted = false;
   // Compensated sums would turn an infinity into NaN: those keep the sum of
@@ -142,7 +143,7 @@ __global__ __launch_bounds__(kWave) void move_cols_kernel(MoveColsArgs A) {
     const bool hv = TWO ? !(is_nan(ha) || is_nan(hb)) : !is_nan(ha);
     const bool tv = TWO ? !(is_nan(ta) || is_nan(tb)) : !is_nan(ta);
     if constexpr (IsMoments<S>::value) {
-      if (!shifted && hv) {
+      if (!shifted && fabs((double)ha) < __builtin_inf() && (!TWO || fabs((double)hb) < __builtin_inf())) {
         ka = ha;
         kb = hb;
         shifted = true;
@@ -204,6 +205,8 @@ __global__ __launch_bounds__(kWave) void move_cols_kernel(MoveColsArgs A) {
                              0)) {
           st = S::zero();
           inf_part = 0.0;
+          ka = kb = T(0);
+          shifted = false;
           const int64_t e = p + u;
           for (int64_t r = e - w + 1 > 0 ? e - w + 1 : 0; r <= e && r < n; ++r)
             step((pa + r * A.lda_r)[lc], TWO ? (pb + r * A.ldb_r)[lc] : T(0), canonical_nan<T>(), T(0));

@@ -366,3 +366,43 @@ def test_move_inner_axis_kept_large_output(gpu_lib, dtype, n, cols):
     assert torch.equal(got.isnan(), want.isnan())
     off = ((got - want).abs() / want.abs()).nan_to_num_(nan=0.0).max().item()
     assert off <= (1.2e-7 if dtype == np.float32 else 4.5e-16)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("func", ["move_var", "move_std", "move_cov", "move_corr"])
+def test_move_inner_axis_kept_first_value_infinite(gpu_lib, func, dtype):
+    """An infinity that comes first (in a series, after leading missing values,
+    before or in a later range of positions) leaves with its window: the
+    outputs of windows without one are those of the series with the infinities
+    missing."""
+    import torch
+
+    import numbagg_amd as nb
+    from numbagg_amd import _lib
+    from oracle import exact
+
+    n, cols, window = 600, 40, 10
+    tc = _lib.query("nbg_move_cols_chunk", _lib.NBG_F32 if dtype == np.float32 else _lib.NBG_F64, 1, n, cols, window)
+    assert 2 * window < tc < n // 4
+    rng = np.random.default_rng(7)
+    x, y = (rng.standard_normal((n, cols)).astype(dtype) + 3 for _ in range(2))
+    for c, (lo, at) in enumerate([(0, 0), (0, 5), (tc - window, tc - window), (tc - window - 3, tc - 4), (tc, tc),
+                                  (tc - window, tc + 2)]):
+        for z, other in ((x, 2 * c), (y, 2 * c + 1)):
+            z[lo:at, other] = np.nan
+            z[at, other] = np.inf if c % 2 else -np.inf
+    x[-1, 20] = np.inf  # the last window
+    args = (x, y) if func in ("move_cov", "move_corr") else (x,)
+    clean = [np.where(np.isinf(z), np.nan, z) for z in args]
+    hit = np.zeros(x.shape, bool)
+    for z in args:
+        for t, c in np.argwhere(np.isinf(z)):
+            hit[t:t + window, c] = True
+    got = getattr(nb, func)(*(torch.from_numpy(z).cuda() for z in args), window=window, min_count=3, axis=0)
+    got = got.cpu().numpy()
+    want = exact.move(func, np.ascontiguousarray(clean[0].T), window, 3,
+                      y=np.ascontiguousarray(clean[-1].T) if len(args) == 2 else None).T
+    ok = ~hit
+    assert np.array_equal(np.isnan(got[ok]), np.isnan(want[ok]))
+    assert_allclose(got[ok], want[ok], rtol=2.4e-7 if dtype == np.float32 else 1e-11,
+                    atol=1e-6 if dtype == np.float32 else 1e-13)
