@@ -72,15 +72,23 @@ __device__ __forceinline__ T cols_out(const typename Traits<T, KIND>::S& s, int6
   if constexpr (sizeof(T) == 8 && Traits<T, KIND>::SHIFT) {
     if (s.c < (KIND == kCorr ? (mc > 1 ? mc : 1) : (mc > 2 ? mc : 2))) return canonical_nan<T>();
     const double c = (double)s.c;
+    // The scaled forms leave the range of float64 sooner than the row kernel's,
+    // which the fallback below is; infinite inputs (NaN here) take it too.
     if constexpr (KIND == kCorr) {
       const double vv = scaled_comoment(c, s.s11, s.s1, s.s1) * scaled_comoment(c, s.s22, s.s2, s.s2);
-      return vv > 0 ? scaled_comoment(c, s.s12, s.s1, s.s2) / sqrt(vv) : canonical_nan<T>();
+      if (__builtin_expect(vv < __builtin_inf(), 1))
+        return vv > 0 ? scaled_comoment(c, s.s12, s.s1, s.s2) / sqrt(vv) : canonical_nan<T>();
     } else if constexpr (KIND == kCov) {
-      return scaled_comoment(c, s.s12, s.s1, s.s2) / (c * (c - 1.0));
+      const double cov = scaled_comoment(c, s.s12, s.s1, s.s2);
+      if (__builtin_expect(fabs(cov) < __builtin_inf(), 1)) return cov / (c * (c - 1.0));
     } else {
-      const double var = scaled_comoment(c, s.s11, s.s1, s.s1) / (c * (c - 1.0));
-      return KIND == kStd ? sqrt(var) : var;
+      const double m2 = scaled_comoment(c, s.s11, s.s1, s.s1);
+      if (__builtin_expect(fabs(m2) < __builtin_inf(), 1)) {
+        const double var = m2 / (c * (c - 1.0));
+        return KIND == kStd ? sqrt(var) : var;
+      }
     }
+    return Traits<T, KIND>::out(s, mc, nullptr);
   } else {
     return Traits<T, KIND>::out(s, mc, nullptr);
   }

@@ -406,3 +406,28 @@ def test_move_inner_axis_kept_first_value_infinite(gpu_lib, func, dtype):
     assert np.array_equal(np.isnan(got[ok]), np.isnan(want[ok]))
     assert_allclose(got[ok], want[ok], rtol=2.4e-7 if dtype == np.float32 else 1e-11,
                     atol=1e-6 if dtype == np.float32 else 1e-13)
+
+
+def test_move_inner_axis_kept_extreme_scales(gpu_lib):
+    """float64 data whose sums of squares lie near the end of the range: the
+    moments that the row kernel gives (shifts of 0 on both sides, so that the
+    row kernel's squared sums of 100 values stay in range)."""
+    import torch
+
+    import numbagg_amd as nb
+    from numbagg_amd import _lib
+
+    rng = np.random.default_rng(2)
+    x, y = (torch.from_numpy(rng.standard_normal((400, 48))).cuda() for _ in range(2))
+    tc = _lib.query("nbg_move_cols_chunk", _lib.NBG_F64, 1, 400, 48, 100)
+    for z in (x, y):  # the first value of each range's first window
+        z[0] = 0
+        z[[t for t in range(-100, 400, tc) if t >= 0 and (t + 100) % tc == 0]] = 0
+    for func, scales in (("move_var", (2e152,)), ("move_std", (2e152,)), ("move_cov", (2e152, 2e152)),
+                         ("move_corr", (2e75, 2e75)), ("move_corr", (1e152, 1.0))):
+        args = [a * s for a, s in zip((x, y), scales)]
+        got = getattr(nb, func)(*args, window=100, min_count=2, axis=0)
+        want = getattr(nb, func)(*(a.t().contiguous() for a in args), window=100, min_count=2, axis=-1).t()
+        assert torch.equal(got.isfinite(), want.isfinite()) and got[1:].isfinite().all(), func
+        assert_allclose(got[1:].cpu().numpy(), want[1:].cpu().numpy(), rtol=1e-11,
+                        atol=1e-11 if func == "move_corr" else 1e-11 * scales[0] * scales[-1], err_msg=func)
