@@ -67,6 +67,16 @@ __device__ __forceinline__ double scaled_comoment(double c, const Comp<double>& 
   return d + (e + (pe - qe));
 }
 
+// The same for a variance, which is zero where all that is left is the rounding
+// of the sums: for one repeated value after others that is up to 2^-92 of
+// c * s11 where both are alike in size, 2^-77 where that value lies nearest to
+// the shift (2000 positions of random values or walks, emulated).
+// Taken for a variance it made correlations of noise.
+__device__ __forceinline__ double scaled_m2(double c, const Comp<double>& s11, const Comp<double>& s1) {
+  const double d = scaled_comoment(c, s11, s1, s1);
+  return fabs(d) <= 0x1p-76 * (c * s11.hi) ? 0.0 : d;
+}
+
 template <typename T, int KIND>
 __device__ __forceinline__ T cols_out(const typename Traits<T, KIND>::S& s, int64_t mc) {
   if constexpr (sizeof(T) == 8 && Traits<T, KIND>::SHIFT) {
@@ -75,14 +85,14 @@ __device__ __forceinline__ T cols_out(const typename Traits<T, KIND>::S& s, int6
     // The scaled forms leave the range of float64 sooner than the row kernel's,
     // which the fallback below is; infinite inputs (NaN here) take it too.
     if constexpr (KIND == kCorr) {
-      const double vv = scaled_comoment(c, s.s11, s.s1, s.s1) * scaled_comoment(c, s.s22, s.s2, s.s2);
+      const double vv = scaled_m2(c, s.s11, s.s1) * scaled_m2(c, s.s22, s.s2);
       if (__builtin_expect(vv < __builtin_inf(), 1))
         return vv > 0 ? scaled_comoment(c, s.s12, s.s1, s.s2) / sqrt(vv) : canonical_nan<T>();
     } else if constexpr (KIND == kCov) {
       const double cov = scaled_comoment(c, s.s12, s.s1, s.s2);
       if (__builtin_expect(fabs(cov) < __builtin_inf(), 1)) return cov / (c * (c - 1.0));
     } else {
-      const double m2 = scaled_comoment(c, s.s11, s.s1, s.s1);
+      const double m2 = scaled_m2(c, s.s11, s.s1);
       if (__builtin_expect(fabs(m2) < __builtin_inf(), 1)) {
         const double var = m2 / (c * (c - 1.0));
         return KIND == kStd ? sqrt(var) : var;

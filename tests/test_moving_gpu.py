@@ -431,3 +431,20 @@ def test_move_inner_axis_kept_extreme_scales(gpu_lib):
         assert torch.equal(got.isfinite(), want.isfinite()) and got[1:].isfinite().all(), func
         assert_allclose(got[1:].cpu().numpy(), want[1:].cpu().numpy(), rtol=1e-11,
                         atol=1e-11 if func == "move_corr" else 1e-11 * scales[0] * scales[-1], err_msg=func)
+
+
+def test_move_inner_axis_kept_constant_windows_f64(gpu_lib):
+    """float64 windows of one repeated value that follow other values have
+    variance exactly zero and no correlation."""
+    import torch
+
+    import numbagg_amd as nb
+
+    rng = np.random.default_rng(6)
+    x = rng.uniform(-500, 500, (600, 200))
+    x[70:] = x[70]
+    y = rng.standard_normal(x.shape)
+    a, b = torch.from_numpy(x).cuda(), torch.from_numpy(y).cuda()
+    assert (nb.move_var(a, window=30, axis=0)[99:] == 0).all()
+    assert (nb.move_std(a, window=30, axis=0)[99:] == 0).all()
+    assert nb.move_corr(a, b, window=30, axis=0)[99:].isnan().all()
