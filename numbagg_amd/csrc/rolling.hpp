@@ -381,11 +381,14 @@ struct Traits<T, kCorr> {
   static constexpr bool SHIFT = true;
   // float32: from c times the (co-)moments about the means, whose factors
   // cancel, so neither 1/c nor a table of it is needed
-  // (c s12 - s1 s2) / sqrt((c s11 - s1^2)(c s22 - s2^2))
+  // (c s12 - s1 s2) / sqrt((c s11 - s1^2)(c s22 - s2^2)).
+  // Both products of a variance are rounded: where the sums of a window of one
+  // value are exact they are equal, and the window has no correlation. (A fused
+  // multiply-add leaves the rounding of s1^2, half of the time positive.)
   __device__ static T from_sums(const S& s, int64_t mce) {
     const double c = (double)s.c, s1 = s.s1.to_double(), s2 = s.s2.to_double();
-    const double va = fma(c, s.s11.to_double(), -(s1 * s1));
-    const double vb = fma(c, s.s22.to_double(), -(s2 * s2));
+    const double va = c * s.s11.to_double() - s1 * s1;
+    const double vb = c * s.s22.to_double() - s2 * s2;
     const double cv = fma(c, s.s12.to_double(), -(s1 * s2));
     const double vv = va * vb;
     const bool in_range = vv > 0x1p-1000 && vv < 0x1p1000;

@@ -448,3 +448,22 @@ def test_move_inner_axis_kept_constant_windows_f64(gpu_lib):
     assert (nb.move_var(a, window=30, axis=0)[99:] == 0).all()
     assert (nb.move_std(a, window=30, axis=0)[99:] == 0).all()
     assert nb.move_corr(a, b, window=30, axis=0)[99:].isnan().all()
+
+
+@pytest.mark.parametrize("axis", [-1, 0])
+def test_move_corr_constant_windows(gpu_lib, axis):
+    """Windows of one repeated value have no correlation, also where that value
+    is not the shift: its sums and sums of squares are exact (24-bit values from
+    a shift of 0, 30 of them)."""
+    import torch
+
+    import numbagg_amd as nb
+
+    rng = np.random.default_rng(5)
+    x = np.repeat(rng.uniform(-500, 500, (64, 1)).astype(np.float32), 200, axis=1)
+    x[:, 0] = 0
+    y = rng.standard_normal(x.shape).astype(np.float32)
+    a, b = (torch.from_numpy(np.ascontiguousarray(z if axis else z.T)).cuda() for z in (x, y))
+    got = nb.move_corr(a, b, window=30, min_count=2, axis=axis).cpu().numpy()
+    got = got if axis else got.T
+    assert np.isnan(got[:, 30:]).all()
