@@ -530,7 +530,7 @@ __global__ __launch_bounds__(kMxThreads) void mx_tiny_kernel(MxStaticArgs a) {
   double P[NPAIR], S[NS], Q[CORR ? NS : 1];
   int cnt[NPAIR];
   double sh[V];
-  bool inf = false;
+  bool over = false;  // an infinite factor of a product with a mask
 #pragma unroll
   for (int k = 0; k < NPAIR; ++k) P[k] = 0.0, cnt[k] = 0;
 #pragma unroll
@@ -588,7 +588,10 @@ __global__ __launch_bounds__(kMxThreads) void mx_tiny_kernel(MxStaticArgs a) {
           ok[v] = __ballot(t == t);
           y[v] = t == t ? (double)t - sh[v] : 0.0;
           m[v] = t == t ? 1.0 : 0.0;
-          inf = inf || fabs((double)t) == __builtin_inf();
+          // a float32 difference is infinite, and its square, only for an
+          // infinite value; float64 squares are looked at below
+          if (sizeof(T) == 4) over = over || fabs((double)t) == __builtin_inf();
+          else if (!CORR) over = over || fabs(y[v]) == __builtin_inf();
         }
         int k = 0;
 #pragma unroll
@@ -599,6 +602,7 @@ __global__ __launch_bounds__(kMxThreads) void mx_tiny_kernel(MxStaticArgs a) {
 #pragma unroll
         for (int i = 0; i < V; ++i) {
           const double q = y[i] * y[i];
+          if (sizeof(T) == 8 && CORR) over = over || q == __builtin_inf();
 #pragma unroll
           for (int j = 0; j < V; ++j) {
             if (j >= i) {
@@ -631,9 +635,9 @@ __global__ __launch_bounds__(kMxThreads) void mx_tiny_kernel(MxStaticArgs a) {
 #pragma unroll
     for (int k = 0; k < NPAIR; ++k) s_cnt[wave][k] = cnt[k];
   }
-  if (__builtin_expect(live && __ballot(inf) != 0ull, 0)) {
-    // An infinity times a missing value's zero was NaN: this wave's sums again,
-    // pair by pair, by selection.
+  if (__builtin_expect(live && __ballot(over) != 0ull, 0)) {
+    // An infinity, or a float64 square beyond the range, times a missing
+    // value's zero was NaN: this wave's sums again, pair by pair, by selection.
 #pragma unroll 1
     for (int ij = 0; ij < V * V; ++ij) {
       const int i = ij / V, j = ij % V;

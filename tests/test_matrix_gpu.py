@@ -478,3 +478,24 @@ def test_static_few_variables_infinities(gpu_lib):
         assert np.isnan(got[b, i, i]) and got[b, i, j] == got[b, j, i]
     assert np.isnan(got[0, 0, 1]) and np.isnan(got[3, 1, 2])
     assert np.isfinite(got[1]).all()
+
+
+@pytest.mark.parametrize("batch,nobs", [(512, 200), (513, 1200)])
+@pytest.mark.parametrize("func", ["nancorrmatrix", "nancovmatrix"])
+def test_static_few_variables_large_values(gpu_lib, func, batch, nobs):
+    """A value whose square leaves the float64 range does not touch the pairs
+    whose other variable is missing there."""
+    import numbagg_amd as nb
+    from oracle import exact
+
+    rng = np.random.default_rng(batch)
+    x = rng.standard_normal((batch, 3, nobs))
+    clean = x.copy()
+    x[0, 0, 10], x[5, 1, nobs - 3] = 1e160, -1e155
+    x[0, 1, 10] = x[5, 2, nobs - 3] = np.nan
+    got = getattr(nb, func)(x)
+    clean[0, :2, 10] = clean[5, 1:, nobs - 3] = np.nan
+    want = exact.matrix(func, clean)
+    for b, i, j in ((0, 0, 1), (5, 1, 2)):
+        assert abs(got[b, i, j] - want[b, i, j]) <= 1e-12 and got[b, i, j] == got[b, j, i], (b, i, j)
+    assert np.isfinite(got[1]).all()
