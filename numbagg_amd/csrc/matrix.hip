@@ -790,12 +790,14 @@ struct PairSums {
   }
   // The output for the current window, in forms scaled by n so that neither
   // needs a division by n: corr = (n sp - si sj) / sqrt((n qi - si^2)(n qj -
-  // sj^2)); cov = (n sp - si sj) / (n (n - 1)).
+  // sj^2)); cov = (n sp - si sj) / (n (n - 1)). Both products of a variance are
+  // rounded: where the sums of a window of one value are exact they are equal
+  // and it is zero, which a fused multiply-add would make the rounding of si^2.
   __device__ __forceinline__ double value(int least, bool diag) const {
     const double dn = (double)n;
-    const double cv = fma(dn, sp, -(si * sj));
     if (CORR) {
-      const double vi = fma(dn, qi, -(si * si)), vj = fma(dn, qj, -(sj * sj));
+      const double cv = fma(dn, sp, -(si * sj));
+      const double vi = dn * qi - si * si, vj = dn * qj - sj * sj;
       const double vv = vi * vj;
       const bool ok = n >= least && vi > 0.0 && vj > 0.0;
       const bool range = vv >= 0x1p-1000 && vv <= 0x1p1000;
@@ -806,6 +808,7 @@ struct PairSums {
     }
     // 1 / (n (n - 1)) by a refined reciprocal, the quotient corrected by its
     // remainder (the rounded one but for rare ties)
+    const double cv = dn * sp - si * sj;
     const double den = n >= 2 ? dn * (dn - 1.0) : 2.0;
     const double e = __builtin_amdgcn_rcp(den);
     const double r = fma(e, fma(-den, e, 1.0), e);

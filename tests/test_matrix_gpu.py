@@ -499,3 +499,20 @@ def test_static_few_variables_large_values(gpu_lib, func, batch, nobs):
     for b, i, j in ((0, 0, 1), (5, 1, 2)):
         assert abs(got[b, i, j] - want[b, i, j]) <= 1e-12 and got[b, i, j] == got[b, j, i], (b, i, j)
     assert np.isfinite(got[1]).all()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_moving_constant_windows(gpu_lib, dtype):
+    """Windows of one repeated value have variance exactly zero and no
+    correlation, also where that value is not the shift (24-bit values from a
+    shift of 0, 30 of them: their sums and sums of squares are exact)."""
+    import numbagg_amd as nb
+
+    rng = np.random.default_rng(4)
+    x = np.repeat(rng.uniform(-500, 500, (1, 16)).astype(np.float32), 64, axis=0).astype(dtype)
+    x[0] = 0
+    x[:, 15] = rng.standard_normal(64)
+    cov = nb.move_covmatrix(x, window=30, min_count=2)
+    corr = nb.move_corrmatrix(x, window=30, min_count=2)
+    assert (cov[30:, :15, :15] == 0).all()
+    assert np.isnan(corr[30:, :15]).all() and np.isnan(corr[30:, :, :15]).all() and (corr[30:, 15, 15] == 1).all()
