@@ -807,13 +807,14 @@ struct PairSums {
       return ok ? r : __builtin_nan("");
     }
     // 1 / (n (n - 1)) by a refined reciprocal, the quotient corrected by its
-    // remainder (the rounded one but for rare ties)
+    // remainder (the rounded one but for rare ties); an infinite quotient has
+    // no remainder and is the result
     const double cv = dn * sp - si * sj;
     const double den = n >= 2 ? dn * (dn - 1.0) : 2.0;
     const double e = __builtin_amdgcn_rcp(den);
     const double r = fma(e, fma(-den, e, 1.0), e);
     const double q = cv * r;
-    const double res = fma(fma(-den, q, cv), r, q);
+    const double res = fabs(q) < __builtin_inf() ? fma(fma(-den, q, cv), r, q) : q;
     return n >= least ? res : __builtin_nan("");
   }
 };

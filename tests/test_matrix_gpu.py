@@ -516,3 +516,27 @@ def test_moving_constant_windows(gpu_lib, dtype):
     corr = nb.move_corrmatrix(x, window=30, min_count=2)
     assert (cov[30:, :15, :15] == 0).all()
     assert np.isnan(corr[30:, :15]).all() and np.isnan(corr[30:, :, :15]).all() and (corr[30:, 15, 15] == 1).all()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_moving_covariance_infinities(gpu_lib, dtype):
+    """A window with an infinity gives what its sums about the first values
+    give: an infinity or NaN by the signs of the other variable's sums."""
+    import numbagg_amd as nb
+
+    rng = np.random.default_rng(9)
+    x = rng.standard_normal((64, 6)).astype(dtype)
+    x[20, 0] = np.inf
+    window = 8
+    got = nb.move_covmatrix(x, window=window, min_count=2)
+    y = x.astype(np.float64) - x[0].astype(np.float64)
+    seen = set()
+    with np.errstate(invalid="ignore"):
+        for t in range(20, 20 + window):
+            w = y[t - window + 1:t + 1]
+            for j in range(1, 6):
+                want = window * (w[:, 0] * w[:, j]).sum() - w[:, 0].sum() * w[:, j].sum()
+                seen.add(str(want))
+                assert np.array_equal(got[t, 0, j], dtype(want), equal_nan=True), (t, j)
+                assert np.array_equal(got[t, j, 0], dtype(want), equal_nan=True), (t, j)
+    assert "nan" in seen and len(seen) > 1  # an infinity of either sign too
