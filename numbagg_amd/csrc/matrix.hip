@@ -40,6 +40,7 @@
 // state and writes the outputs. Shifts are per variable over the whole series.
 #include <cmath>
 #include <initializer_list>
+#include <limits>
 #include <type_traits>
 
 #include "common.hpp"
@@ -770,11 +771,12 @@ struct MoveState {
 };
 
 // Window sums of one pair. Observations enter and leave without branches: an
-// invalid pair becomes the shifts (two selects of T), zeros after them.
-template <typename T, bool CORR>
+// invalid pair becomes the shifts (two selects of T), zeros after them. N: the
+// type of the count of pairs, which a window of that many steps may reach.
+template <typename T, bool CORR, typename N>
 struct PairSums {
   double si = 0.0, sj = 0.0, sp = 0.0, qi = 0.0, qj = 0.0;
-  int n = 0;
+  N n = 0;
   template <bool SUB>
   __device__ __forceinline__ void add(T xi, T xj, T ti, T tj, double ci, double cj) {
     const bool both = !__builtin_isunordered(xi, xj);
@@ -786,14 +788,14 @@ struct PairSums {
       qi = fma(SUB ? -yi : yi, yi, qi);
       qj = fma(SUB ? -yj : yj, yj, qj);
     }
-    n += SUB ? -(int)both : (int)both;
+    n += SUB ? -(N)both : (N)both;
   }
   // The output for the current window, in forms scaled by n so that neither
   // needs a division by n: corr = (n sp - si sj) / sqrt((n qi - si^2)(n qj -
   // sj^2)); cov = (n sp - si sj) / (n (n - 1)). Both products of a variance are
   // rounded: where the sums of a window of one value are exact they are equal
   // and it is zero, which a fused multiply-add would make the rounding of si^2.
-  __device__ __forceinline__ double value(int least, bool diag) const {
+  __device__ __forceinline__ double value(N least, bool diag) const {
     const double dn = (double)n;
     if (CORR) {
       const double cv = fma(dn, sp, -(si * sj));
@@ -857,9 +859,12 @@ __global__ __launch_bounds__(kMxThreads) void mx_move_kernel(MxMoveArgs a) {
   const double cj = a.shift[(b * a.tiles + tile) * a.nv + j];
   const T ti = (T)ci, tj = (T)cj;  // exact: shifts are values of the data
   const bool diag = i == j;
-  const int least = a.min_count > 2 ? (a.min_count < 0x7fffffff ? (int)a.min_count : 0x7fffffff) : 2;
+  // counts of pairs: a series of 2^31 steps or more has offsets of 64 bits
+  using N = typename std::conditional<sizeof(IT) == 4, int, int64_t>::type;
+  constexpr int64_t most = std::numeric_limits<N>::max();
+  const N least = a.min_count > 2 ? (N)(a.min_count < most ? a.min_count : most) : 2;
   const IT step = (IT)a.nv, ostep = (IT)np, back = (IT)(a.window * a.nv);
-  PairSums<T, CORR> st;
+  PairSums<T, CORR, N> st;
   IT oi = (IT)(t_w * a.nv + i), oj = (IT)(t_w * a.nv + j);
   int64_t t = t_w;
   for (; t < t_start; ++t, oi += step, oj += step) st.template add<false>(x[oi], x[oj], ti, tj, ci, cj);
