@@ -729,12 +729,14 @@ StaticPlan static_plan(int64_t batch, int64_t nv, int64_t nobs, bool corr) {
   p.tiles = p.ntile * (p.ntile + 1) / 2;
   const int64_t items = batch * p.tiles;
   // Whole rounds of waves: at most the target, so no last round runs a few;
-  // short spans only up to kStaticFineWaves.
+  // short spans only up to kStaticFineWaves (or a lower NBG_MATRIX_WAVES).
   const int64_t n = items > 0 ? items : 1;
-  int64_t splits = knob("NBG_MATRIX_WAVES", kStaticTargetWaves) / n;
+  const int64_t target = knob("NBG_MATRIX_WAVES", kStaticTargetWaves);
+  int64_t splits = target / n;
   const int64_t coarse = (nobs + kStaticSpan - 1) / kStaticSpan, fine = (nobs + kStaticMinSpan - 1) / kStaticMinSpan;
   if (splits > coarse) splits = coarse;
-  const int64_t more = kStaticFineWaves / n < fine ? kStaticFineWaves / n : fine;
+  int64_t more = (target < kStaticFineWaves ? target : kStaticFineWaves) / n;
+  if (more > fine) more = fine;
   if (splits < more) splits = more;
   if (splits < 1) splits = 1;
   int64_t span = (nobs + splits - 1) / splits;

@@ -91,3 +91,12 @@ def test_applied_sets_recorded_knobs(lib, tmp_path, monkeypatch):
                 assert lib.nbg_tune_get(b"NBG_GROUP_ROWS", 2) == 1
     finally:
         plain_tuning.reload_database()
+
+
+def test_matrix_waves_bounds_the_splits(lib, monkeypatch):
+    """NBG_MATRIX_WAVES is the number of waves that static matrices are split
+    for: one wave leaves no partial sums in the workspace."""
+    default = _lib.query("nbg_matrix_workspace_bytes", 1, 20, 5000)
+    monkeypatch.setenv("NBG_MATRIX_WAVES", "1")
+    one = _lib.query("nbg_matrix_workspace_bytes", 1, 20, 5000)
+    assert one == (20 * 8 + 255) // 256 * 256 and default > one
