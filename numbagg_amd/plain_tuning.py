@@ -136,11 +136,12 @@ class PlainTuningDB:
         """``get`` of this device's shape class, without building its key each
         time (one entry per class seen: log2 sizes, so a few thousand at most)."""
         at = (func, dtype, rows.bit_length(), n.bit_length(), extra.bit_length())
+        found = self._lookups  # taken before the entry is read: ``put`` records first and replaces this then
         try:
-            return self._lookups[at]
+            return found[at]
         except KeyError:
             knobs = self.get(shape_key(device_arch(), func, str(dtype), rows, n, extra)) or None
-            self._lookups[at] = knobs
+            found[at] = knobs
             return knobs
 
     def put(self, key: str, knobs: dict, timings: dict) -> None:

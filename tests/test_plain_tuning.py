@@ -100,3 +100,22 @@ def test_matrix_waves_bounds_the_splits(lib, monkeypatch):
     monkeypatch.setenv("NBG_MATRIX_WAVES", "1")
     one = _lib.query("nbg_matrix_workspace_bytes", 1, 20, 5000)
     assert one == (20 * 8 + 255) // 256 * 256 and default > one
+
+
+def test_lookup_sees_settings_recorded_meanwhile(tmp_path, monkeypatch):
+    """A setting recorded while another thread looks its class up is applied
+    from then on."""
+    monkeypatch.setattr(plain_tuning, "_arch", "gfx950")
+    db = plain_tuning.PlainTuningDB(tmp_path / "db.json")
+    key = plain_tuning.shape_key("gfx950", "move_mean", "float32", 256, 2_000_000, 1000)
+    get = db.get
+
+    def get_then_put(k):
+        found = get(k)
+        monkeypatch.setattr(db, "get", get)
+        db.put(key, {"NBG_MOVE_SPAN": 4}, {"{}": 1.0})
+        return found
+
+    monkeypatch.setattr(db, "get", get_then_put)
+    assert db.lookup("move_mean", "float32", 256, 2_000_000, 1000) is None
+    assert db.lookup("move_mean", "float32", 256, 2_000_000, 1000) == {"NBG_MOVE_SPAN": 4}
