@@ -281,3 +281,23 @@ def test_exp_scalar_alpha_constant_rows(gpu_lib):
     for func in ("move_exp_nanvar", "move_exp_nanstd"):
         got = getattr(nb, func)(x, alpha=0.1)
         assert np.isnan(got[:, 0]).all() and (got[:, 2:] == 0).all()
+
+
+@pytest.mark.parametrize("two_pass", ["0", "1"])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("alpha,mw", [(0.05, 0), (0.3, 0.2), (0.002, 0)])
+def test_exp_std_is_the_root_of_var(gpu_lib, monkeypatch, dtype, two_pass, alpha, mw):
+    """std is the square root of var, to within one unit of the last place. (In
+    one pass, rows of one tile: the carry between tiles is summed in an order
+    that depends on the timing, so two calls differ in their last digits.)"""
+    import numbagg_amd as nb
+
+    monkeypatch.setenv("NBG_EXP_TWO_PASS", two_pass)
+    x = walk_array(20 if two_pass == "0" else 4, 4000 if two_pass == "0" else 20_000, seed=11, dtype=dtype, offset=50.0)
+    var = nb.move_exp_nanvar(x, alpha=alpha, min_weight=mw)
+    std = nb.move_exp_nanstd(x, alpha=alpha, min_weight=mw)
+    assert np.array_equal(np.isnan(var), np.isnan(std))
+    ok = var > 0
+    assert ok.sum() > 70_000
+    root = np.sqrt(var[ok])
+    assert (np.abs(std[ok] - root) <= np.spacing(root)).all()
