@@ -765,57 +765,57 @@ struct UniSpec {
   static constexpr bool SEEN = MOM || KIND == kESum;
 };
 
-// seen: valid observations, saturating at 2 (bits 0-1), and what an infinity
-// among them left in the sums for good: kInfPlus, kInfMinus or both (NaN).
-// Across chunks only these bits carry it (the sums are then finite), as a decay
-// that underflows to 0 would turn an infinity into NaN.
+// seen: valid observations, saturating at 2 (bits 0-1), and for each sum what
+// an infinity in it (an observation's, or a product's beyond the range) leaves
+// for good: bit 2 + 2 c for +inf, 3 + 2 c for -inf, both for NaN. Across chunks
+// only these bits carry it (the sums are then finite), as a decay that
+// underflows to 0 would turn an infinity into NaN. Chunks hold an even number
+// of positions, so a negative decay does not change its sign.
 template <int NS>
 struct UState {
   double b[NS];
   int seen;
 };
-constexpr int kInfPlus = 4, kInfMinus = 8, kInfBoth = 12;
+constexpr int kSeenCount = 3;
 
 __device__ __forceinline__ int join_seen(int a, int b) {
-  return min(2, (a & 3) + (b & 3)) | ((a | b) & kInfBoth);
+  return min(2, (a & kSeenCount) + (b & kSeenCount)) | ((a | b) & ~kSeenCount);
 }
 
-// Infinities and NaN of a chunk's sums (components 0 and, for the moment kinds,
-// all sums of observations) moved into its bits.
+// The sums of a chunk that observations can make infinite: the first for mean
+// and sum, all for the moment kinds.
+template <int KIND, int NS>
+constexpr int inf_sums() {
+  return KIND == kECount ? 0 : (KIND >= kEVar ? NS : 1);
+}
+
+// Infinities and NaN of a chunk's sums moved into its bits.
 template <int KIND, int NS>
 __device__ __forceinline__ void park_inf(UState<NS>& s) {
-  constexpr bool MOM = KIND >= kEVar;
-  if constexpr (KIND == kECount) return;
-  if constexpr (!MOM) {
-    if (__builtin_expect(!isfinite(s.b[0]), 0)) {
-      s.seen |= s.b[0] > 0 ? kInfPlus : (s.b[0] < 0 ? kInfMinus : kInfBoth);
-      s.b[0] = 0.0;
-    }
-  } else {
-    bool ok = true;
+  bool ok = true;
 #pragma unroll
-    for (int c = 0; c < NS; ++c) ok = ok && isfinite(s.b[c]);
-    if (__builtin_expect(!ok, 0)) {
-      s.seen |= kInfBoth;
+  for (int c = 0; c < inf_sums<KIND, NS>(); ++c) ok = ok && isfinite(s.b[c]);
+  if (__builtin_expect(!ok, 0)) {
 #pragma unroll
-      for (int c = 0; c < NS; ++c) s.b[c] = isfinite(s.b[c]) ? s.b[c] : 0.0;
+    for (int c = 0; c < inf_sums<KIND, NS>(); ++c) {
+      const double v = s.b[c];
+      if (!isfinite(v)) {
+        s.seen |= (v > 0 ? 1 : (v < 0 ? 2 : 3)) << (2 + 2 * c);
+        s.b[c] = 0.0;
+      }
     }
   }
 }
 // The sums as the recurrence would hold them.
 template <int KIND, int NS>
 __device__ __forceinline__ void unpark_inf(UState<NS>& s) {
-  constexpr bool MOM = KIND >= kEVar;
-  if (KIND == kECount || __builtin_expect((s.seen & kInfBoth) == 0, 1)) return;
-  const double v = (s.seen & kInfBoth) == kInfPlus    ? __builtin_inf()
-                   : (s.seen & kInfBoth) == kInfMinus ? -__builtin_inf()
-                                                      : __builtin_nan("");
-  s.b[0] = MOM ? __builtin_nan("") : v;
-  if constexpr (MOM) {
-    s.b[1] = __builtin_nan("");
-    if constexpr (KIND == kECov || KIND == kECorr) s.b[2] = __builtin_nan("");
+  if (KIND == kECount || __builtin_expect((s.seen & ~kSeenCount) == 0, 1)) return;
+#pragma unroll
+  for (int c = 0; c < inf_sums<KIND, NS>(); ++c) {
+    const int t = (s.seen >> (2 + 2 * c)) & 3;
+    if (t) s.b[c] = t == 1 ? __builtin_inf() : (t == 2 ? -__builtin_inf() : __builtin_nan(""));
   }
-  s.seen &= 3;
+  s.seen &= kSeenCount;
 }
 
 // later after `earlier` decayed over later's positions (q = d^positions).

@@ -301,3 +301,29 @@ def test_exp_std_is_the_root_of_var(gpu_lib, monkeypatch, dtype, two_pass, alpha
     assert ok.sum() > 70_000
     root = np.sqrt(var[ok])
     assert (np.abs(std[ok] - root) <= np.spacing(root)).all()
+
+
+@pytest.mark.parametrize("two_pass", ["0", "1"])
+@pytest.mark.parametrize("func", ["move_exp_nanmean", "move_exp_nansum", "move_exp_nanvar", "move_exp_nanstd",
+                                  "move_exp_nancov", "move_exp_nancorr"])
+def test_exp_scalar_alpha_infinite_sums(gpu_lib, monkeypatch, func, two_pass):
+    """Sums that an observation or its square makes infinite stay so in every
+    position that follows, whatever thread or tile it falls to: where the
+    outputs are not finite they are those of an array of alphas."""
+    import numbagg_amd as nb
+
+    monkeypatch.setenv("NBG_EXP_TWO_PASS", two_pass)
+    rng = np.random.default_rng(3)
+    n, alpha = 9000, 0.02
+    x, y = (rng.standard_normal((6, n)) for _ in range(2))
+    x[0, 37], x[1, 4100], x[2, 500] = np.inf, -np.inf, 1e160
+    x[3, 70], x[3, 2100], y[4, 15], y[5, 77] = np.inf, -np.inf, np.inf, -1e160
+    two = func in ("move_exp_nancov", "move_exp_nancorr")
+    args = (x, y) if two else (x,)
+    with np.errstate(all="ignore"):
+        got = getattr(nb, func)(*args, alpha=alpha)
+        want = getattr(nb, func)(*args, alpha=np.full(n, alpha))
+    bad = ~np.isfinite(want)
+    assert bad.any()
+    assert np.array_equal(got[bad], want[bad], equal_nan=True)
+    assert np.isfinite(got[~bad]).all()
