@@ -327,3 +327,33 @@ def test_exp_scalar_alpha_infinite_sums(gpu_lib, monkeypatch, func, two_pass):
     assert bad.any()
     assert np.array_equal(got[bad], want[bad], equal_nan=True)
     assert np.isfinite(got[~bad]).all()
+
+
+@pytest.mark.parametrize("two_pass", ["0", "1", ""])
+@pytest.mark.parametrize("func", ["move_exp_nanvar", "move_exp_nanstd", "move_exp_nancov", "move_exp_nancorr"])
+@pytest.mark.parametrize("rows,n,alpha", [(2, 16_385, 0.01), (1, 300_001, 0.02), (40, 30_000, 0.2)])
+def test_exp_scalar_alpha_moments_to_local_scale(gpu_lib, monkeypatch, func, rows, n, alpha, two_pass):
+    """Rows of many tiles against the exact recurrence, to 1e-9 of the moment's
+    own scale: sqrt(var_a var_b) at that position (1 for the correlation)."""
+    import numbagg_amd as nb
+    from oracle import exact
+
+    monkeypatch.setenv("NBG_EXP_TWO_PASS", two_pass)
+    x = walk_array(rows, n, seed=n, offset=5.0)
+    y = walk_array(rows, n, seed=n + 1, offset=-3.0)
+    two = func in ("move_exp_nancov", "move_exp_nancorr")
+    got = getattr(nb, func)(*((x, y) if two else (x,)), alpha=alpha)
+    want = exact.move_exp(func, x, alpha, y=y if two else None, loop_dtype=np.float64)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    if func == "move_exp_nancorr":
+        scale = np.ones_like(want)
+    elif func == "move_exp_nancov":
+        scale = np.sqrt(np.abs(exact.move_exp("move_exp_nancov", x, alpha, y=np.where(np.isnan(y), y, x),
+                                              loop_dtype=np.float64)
+                               * exact.move_exp("move_exp_nancov", y, alpha, y=np.where(np.isnan(x), x, y),
+                                                loop_dtype=np.float64)))
+    else:
+        scale = np.abs(want)
+    ok = ~np.isnan(want)
+    err = np.abs(got[ok] - want[ok]) / np.maximum(scale[ok], 1e-3)
+    assert (err <= 1e-9).all(), err.max()
