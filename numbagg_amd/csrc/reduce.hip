@@ -81,10 +81,14 @@ __device__ __forceinline__ unsigned long long ext_key(T v, bool minimum) {
   return minimum ? ~k : k;
 }
 
-// 1/v for v >= 1: the hardware estimate refined by one Newton step.
-__device__ __forceinline__ double recip_refined(double v) {
-  const double r = __builtin_amdgcn_rcp(v);
-  return fma(r, fma(-v, r, 1.0), r);
+// a / b for a count b >= 1: the hardware's reciprocal (2^-24) refined by one
+// Newton step (2^-48: 9e-16 for 255, 2e-15 for 4095), the quotient corrected by
+// its exact remainder.
+__device__ __forceinline__ double div_small(double a, double b) {
+  const double e = __builtin_amdgcn_rcp(b);
+  const double r = fma(e, fma(-b, e, 1.0), e);
+  const double q = a * r;
+  return fma(fma(-b, q, a), r, q);
 }
 
 // (count, mean, M2) and Chan's merge of another such triple.
@@ -195,10 +199,9 @@ struct Lane {
     ch.merge((double)nb, mb, m2b);
   }
 
-  // The same without float64 divisions: the batch mean from a refined
-  // reciprocal corrected by its remainder (so equal values have exactly their
-  // value as mean, and no variance), the merge's weight from a refined
-  // reciprocal (about 1 ULP).
+  // The same without float64 divisions: the batch mean and the merge's weight
+  // by reciprocals (div_small), whose quotients are the rounded ones but for
+  // rare ties; so equal values have exactly their value as mean, and no variance.
   template <int B>
   __device__ __forceinline__ void fold_batch_rcp(const T (&v)[B]) {
     double sb = 0.0;
@@ -210,9 +213,7 @@ struct Lane {
       nb += valid ? 1 : 0;
     }
     const double dn = (double)nb;
-    const double r = recip_refined(nb > 0 ? dn : 1.0);
-    const double q = sb * r;
-    const double mb = fma(fma(-dn, q, sb), r, q);
+    const double mb = div_small(sb, nb > 0 ? dn : 1.0);
     double m2b = 0.0;
 #pragma unroll
     for (int j = 0; j < B; ++j) {
@@ -226,7 +227,7 @@ struct Lane {
     }
     const double tot = ch.n + dn;
     const double d = mb - ch.mean;
-    const double f = dn * recip_refined(tot);
+    const double f = div_small(dn, tot);
     ch.mean += d * f;
     ch.m2 += m2b + d * d * ch.n * f;
     ch.n = tot;

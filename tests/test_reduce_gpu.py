@@ -366,3 +366,19 @@ def test_inner_axis_kept_special_values(gpu_lib):
     at = nb.nanargmax(t[:, 6:], axis=0)
     assert not at.any()
     assert nb.nanargmin(t[:, 3:6], axis=0).tolist() == [0, 20, 0]
+
+
+def test_inner_axis_kept_variance_weights(gpu_lib):
+    """Each lane merges 248 zeros and 7 ones, a mean of 7 / 255, equal in all
+    lanes: the variance over an outer axis is 128 lanes times 248 * 7 / 255, to
+    four roundings (the weight, two products with it, the division)."""
+    import torch
+
+    import numbagg_amd as nb
+
+    lane = torch.cat([torch.zeros(248), torch.tensor([np.nan]), torch.ones(7)])
+    x = lane.double().repeat_interleave(128).cuda()  # 128 row lanes: rows k, k + 128, ...
+    t = x[None, :, None].expand(2048, -1, 2).contiguous()
+    got = nb.nanvar(t, axis=1)
+    want = 128 * 248 * 7 / 255 / (128 * 255 - 1)
+    assert ((got - want).abs() <= 4 * 2.0**-53 * want).all()
