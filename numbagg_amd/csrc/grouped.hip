@@ -1038,7 +1038,10 @@ int group_impl(GArgs a, int strategy, void* ws, size_t ws_bytes, hipStream_t s) 
       return launch_finalize<TV, KIND>(a, nullptr, s);
     default: {  // var / std
       if constexpr (std::is_floating_point<TV>::value) {
-        if (lds) {
+        // Slices of float64 labels take the two passes below: a label whose
+        // first value lies far from the others (100 deviations: 2e-12 of the
+        // variance) keeps its digits, which a float32 result does not show.
+        if (lds && !(a.sliced && sizeof(TV) == 8)) {
           // One pass: per-(row, label) shifted moments in LDS, moved to a
           // global shift per (row, label) when each workgroup flushes them.
           if ((rc = launch_init(acc0, 0ull, acc1, 0ull, per, s))) return rc;
@@ -1052,7 +1055,7 @@ int group_impl(GArgs a, int strategy, void* ws, size_t ws_bytes, hipStream_t s) 
           return launch_finalize<TV, KIND>(a, nullptr, s);
         }
       }
-      // Global accumulators: per-label means, then squared deviations.
+      // Global accumulators (or slices): per-label means, then squared deviations.
       // The float64 means come from float64 sums, so the deviations' own sum
       // (the usual two-pass correction term) is negligible: with n values
       // per label its share of sum d^2 is about (n 2**-53 |mean| / std)^2.

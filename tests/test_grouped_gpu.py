@@ -447,3 +447,24 @@ def test_label_slices(gpu_lib, monkeypatch, dtype, ldt, num_labels):
             np.testing.assert_allclose(g, w, rtol=2.4e-7 if dtype == np.float32 else 1e-12, atol=1e-12, err_msg=name)
         else:
             assert np.array_equal(g, w, equal_nan=True), name
+
+
+@pytest.mark.parametrize("rows,num_labels,m", [(64, 9000, 300), (128, 5001, 150)])
+def test_label_slices_variance_of_outlying_first_values(gpu_lib, monkeypatch, rows, num_labels, m):
+    """float64 variances of sliced labels are two-pass ones: a label whose first
+    value lies 100 deviations from the others keeps its digits, also where one
+    workgroup reduces the whole row (a sum of m squares is within sqrt(m)
+    roundings in the mean, 8 sqrt(m) at most)."""
+    import torch
+
+    import numbagg_amd as nb
+
+    monkeypatch.setenv("NBG_GROUP_BLOCKS_PER_CU", "1")
+    g = torch.Generator(device="cuda").manual_seed(m)
+    x = torch.randn(rows, m, num_labels, generator=g, device="cuda", dtype=torch.float64)
+    x[:, 0] += 100.0
+    lab = torch.arange(num_labels, device="cuda").repeat(m)
+    got = nb.group_nanvar(x.view(rows, -1), lab, num_labels=num_labels, axis=-1)
+    want = ((x - x.mean(dim=1, keepdim=True)) ** 2).sum(dim=1) / (m - 1)
+    err = ((got - want) / want).abs().max().item()
+    assert err <= 8 * m**0.5 * 2.0**-53, err
