@@ -313,6 +313,7 @@ struct ExpArgs {
   // scalar alpha: d = 1 - alpha, its square, and d^(K 2^i), the decay over 2^i
   // threads' positions, i = 0..7 (7: half a tile), d^TILE
   double d, d2, pw[8], ptile;
+  double phalf;  // d^(K / 2)
 };
 
 // Stage tile tk of a row in LDS (coalesced across the workgroup; NaN past the
@@ -974,6 +975,7 @@ __global__ __launch_bounds__(kExpThreads) void exp_uni_kernel(ExpArgs A) {
   using Sp = UniSpec<KIND, WT>;
   constexpr int NS = Sp::NS, SW2 = Sp::SW2;
   constexpr int K = uni_items<TX, KIND>();
+  constexpr bool HALVES = K > exp_items<TX, KIND>();  // twice the positions: see the re-run
   constexpr int TILE = kExpThreads * K;
   using St = UState<NS>;
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -1035,11 +1037,20 @@ __global__ __launch_bounds__(kExpThreads) void exp_uni_kernel(ExpArgs A) {
 #pragma unroll
   for (int c = 0; c < NS; ++c) zero.b[c] = 0.0;
   zero.seen = 0;
-  St m = zero;
+  St m = zero, first = zero;  // first: the first half's
 #pragma unroll
-  for (int j = 0; j < K; ++j) step(m, j);
+  for (int j = 0; j < K; ++j) {
+    if (HALVES && j == K / 2) {
+      m.seen = min(2, m.seen);
+      park_inf<KIND>(m);
+      first = m;
+      m = zero;
+    }
+    step(m, j);
+  }
   m.seen = min(2, m.seen);
   park_inf<KIND>(m);
+  if (HALVES) m = uni_join<NS, SW2>(first, m, A.phalf);
 
   // 2. wave scan: within 16-lane rows the earlier range is 2^i threads long
   //    where it exists; the broadcasts join it to the lanes' own prefixes.
@@ -1168,12 +1179,24 @@ __global__ __launch_bounds__(kExpThreads) void exp_uni_kernel(ExpArgs A) {
   }
   if constexpr (MODE == 0) __syncthreads();
 
-  // 4. re-run this thread's positions from its incoming state.
+  // 4. re-run this thread's positions from its incoming state. The second half
+  //    starts from the joined sums again, as a thread of its own would: nearly
+  //    constant data round alike at each position, and 32 in a row are off by
+  //    half as much again as 16 (an infinity stays with the recurrence).
   St s = uni_join<NS, SW2>(s_in, excl, px);
   unpark_inf<KIND>(s);
+  const St start = s;
   TA res[K];
 #pragma unroll
   for (int j = 0; j < K; ++j) {
+    if (HALVES && j == K / 2) {
+      const bool finite = isfinite(s.b[0]) && isfinite(s.b[1]);
+#pragma unroll
+      for (int c = 0; c < NS; ++c) {
+        const double q = c == SW2 ? A.phalf * A.phalf : A.phalf;
+        s.b[c] = finite ? fma(q, start.b[c], first.b[c]) : s.b[c];
+      }
+    }
     step(s, j);
     res[j] = (TA)uni_out<KIND, WT>(s, A.min_weight);
   }
@@ -1389,7 +1412,10 @@ int exp_launch(ExpArgs a, void* ws, size_t ws_bytes, hipStream_t s) {
     a.d = 1.0 - alpha;
     a.d2 = a.d * a.d;
     long double q = 1.0L;  // powers rounded once each
-    for (int i = 0; i < K; ++i) q *= (long double)a.d;
+    for (int i = 0; i < K; ++i) {
+      if (i == K / 2) a.phalf = (double)q;
+      q *= (long double)a.d;
+    }
     for (int i = 0; i < 8; ++i, q *= q) a.pw[i] = (double)q;
     a.ptile = (double)q;
     static_assert(kExpThreads == 256, "2^8 threads per tile");
