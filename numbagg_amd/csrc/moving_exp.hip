@@ -893,7 +893,7 @@ __device__ __forceinline__ double uni_out(const UState<UniSpec<KIND, WT>::NS>& s
   if constexpr (KIND == kECount) return heavy ? b[0] : nan;
   if constexpr (KIND == kESum) return heavy && s.seen ? b[0] : nan;
   if constexpr (KIND == kEMean) {
-    const double m = recip_range(b[1]) && div_range(b[0]) ? fast_div(b[0], b[1]) : b[0] / b[1];
+    const double m = b[0] / b[1];
     return heavy ? m : nan;
   }
   if constexpr (Sp::MOM) {
