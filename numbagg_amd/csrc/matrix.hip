@@ -64,8 +64,8 @@ __device__ __forceinline__ T mx_nan() {
 // in their registers between iterations.
 __device__ __forceinline__ int mx_wave_id() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
 
-// 1/sqrt(v) from the hardware estimate and one Newton step (about 1 ULP of
-// float64), for v within [2^-1000, 2^1000].
+// 1/sqrt(v) from the hardware estimate (2^-24) and one Newton step (4e-15 off at
+// most), for v within [2^-1000, 2^1000].
 __device__ __forceinline__ double mx_rsqrt(double v) {
   const double y = __builtin_amdgcn_rsq(v);
   return y * fma(-(0.5 * v) * y, y, 1.5);

@@ -13,7 +13,8 @@
 // Each lane walks its own column: the window ending before the range is summed
 // first, then every position adds its head and removes its tail (`window`
 // positions back, read again: those lines were fetched `window` steps ago and
-// come from the L2 or the MALL). All loads are whole 256-byte lines of a wave,
+// come from the L2 or the MALL). An infinity that leaves makes the lane sum its
+// window anew. All loads are whole 256-byte lines of a wave,
 // and the next 16 positions are in flight while 8 are evaluated.
 // Outputs turn through LDS, one 128-byte line of each of the 64 series at a
 // time, and leave as whole lines past the caches: each series is written up to
@@ -278,10 +279,11 @@ __global__ __launch_bounds__(kWave) void move_cols_kernel(MoveColsArgs A) {
 
 // Positions per wave, or 0 where the general path is the better one: fewer
 // than half a wave of columns, or a window that would be summed anew (and its
-// tails read) for too few positions. About 8192 waves (8 per SIMD) where the
-// array holds that many of at least 64 positions; at most 4096 positions (2048
-// for float64), after which the running sums start afresh, as the tiles of
-// moving.hip do.
+// tails read) for too few positions. A grid of about 8192 waves where the array
+// holds that many of at least 64 positions (LDS lets a CU hold 9 of them at a
+// time where whole lines are written, else 19: about half of the grid, so that
+// the rest evens out the end); at most 4096 positions (2048 for float64), after
+// which the running sums start afresh, as the tiles of moving.hip do.
 int64_t move_cols_chunk(int elem, int64_t outer, int64_t n, int64_t cols, int64_t window) {
   if (outer <= 0 || n <= 0 || cols < 32 || window <= 0) return 0;
   const int64_t groups = (cols + kWave - 1) / kWave;

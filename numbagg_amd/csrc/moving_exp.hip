@@ -196,8 +196,8 @@ __device__ __forceinline__ void exp_step(double* s, int& seen, double a, double 
   }
 }
 
-// Division by a shared reciprocal. r: 1/b from the hardware estimate
-// refined by one Newton step (about 1 ULP of float64); div_rn then corrects
+// Division by a shared reciprocal. r: 1/b from the hardware estimate (2^-24)
+// refined by one Newton step (2^-48); div_rn then corrects
 // a * r with the exact remainder a - b * (a * r) from one fused multiply-add,
 // which gives the correctly rounded quotient a / b (the reference's division)
 // except in rare near-tie cases, where it is 1 ULP off. Valid while
@@ -212,7 +212,8 @@ __device__ __forceinline__ double div_rn(double a, double b, double r) {
 }
 __device__ __forceinline__ bool div_range(double x) { return fabs(x) <= 0x1p500; }
 __device__ __forceinline__ bool recip_range(double b) { return fabs(b) >= 0x1p-500 && fabs(b) <= 0x1p500; }
-// 1/sqrt(v) for v in [2**-1000, 2**1000]: estimate plus one Newton step.
+// 1/sqrt(v) for v in [2**-1000, 2**1000]: estimate plus one Newton step (up to
+// 4e-15 off: for correlations, whose own cancellation is larger).
 __device__ __forceinline__ double rsqrt_refined(double v) {
   const double y = __builtin_amdgcn_rsq(v);
   return y * fma(-(0.5 * v) * y, y, 1.5);
@@ -275,22 +276,21 @@ __device__ __forceinline__ double exp_out(const double* s, int seen, double mw) 
   return (vv >= 0x1p-1000 && vv <= 0x1p1000) ? cov * rsqrt_refined(vv) : cov / sqrt(vv);
 }
 
-
 // Positions per thread: 64 bytes of input; 32 float32 positions for the
 // kinds with small maps (count, mean, sum: twice as many positions per tile,
 // half as many look-back hops per row). Measured on MI355X for float32
-// (256, 2M), alpha 0.01, 16 -> 32 positions: mean 2.06 -> 1.77 ms, sum /
-// count 1.99 / 2.00 -> 1.62 / 1.61 ms; var 2.51 -> 3.06 ms and corr 3.16 ->
-// 4.37 ms, so the moment kinds keep 16.
+// (256, 2M), alpha 0.01, 16 -> 32 positions in exp_kernel: mean 2.06 -> 1.77
+// ms, sum / count 1.99 / 2.00 -> 1.62 / 1.61 ms; var 2.51 -> 3.06 ms and corr
+// 3.16 -> 4.37 ms, so the moment kinds keep 16 there.
 template <typename TX, int KIND>
 constexpr int exp_items() {
   return (sizeof(TX) == 4 && ExpSpec<KIND>::NS <= 3) ? 32 : 64 / (int)sizeof(TX);
 }
 
 // Positions per thread of exp_uni_kernel: its var / std states are small enough
-// for twice the positions (float32 (256, 2M) nanvar 16 -> 32 positions 1463 ->
-// 1328 us, float64 (200, 300k) 8 -> 16 260 -> 237 us; corr 680 -> 782 and 402 ->
-// 473 us, mean of float64 unchanged).
+// for twice the positions, in two halves with sums of their own (float32 (256,
+// 2M) nanvar 16 -> 32 positions 1463 -> 1311 us, float64 (200, 300k) 8 -> 16 260
+// -> 237 us; corr 680 -> 782 and 402 -> 473 us, mean of float64 unchanged).
 template <typename TX, int KIND>
 constexpr int uni_items() {
   return (KIND == kEVar || KIND == kEStd) ? 128 / (int)sizeof(TX) : exp_items<TX, KIND>();
@@ -747,8 +747,8 @@ __global__ __launch_bounds__(kExpThreads) void exp_kernel(ExpArgs A) {
 //
 // Bound by float64 arithmetic for the moment kinds, by HBM for the others.
 // Measured on MI355X for float32 (256, 2M), alpha 0.01 -> float64: nanvar
-// 1.33 ms (6.1 GB: 4.6 TB/s; 66 VALU instructions per position at 16 positions
-// per thread), 2.39 ms in the general kernel with its alpha fixed.
+// 1.31 ms (6.1 GB: 4.7 TB/s), nanstd 1.41 ms, 2.39 and 2.56 ms in the general
+// kernel with its alpha fixed; (256, 1M) nanmean 0.635 ms, nancov 1.05 ms.
 // ---------------------------------------------------------------------------
 template <int KIND, bool WT>
 struct UniSpec {

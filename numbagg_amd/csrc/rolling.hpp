@@ -225,8 +225,8 @@ __device__ __forceinline__ void acc_moments(MomStats<T, NM>& s, bool valid, T a,
   }
 }
 
-// 1/c for a positive count: hardware reciprocal plus one Newton step (about
-// 1 ULP of float64, far below the float32 rounding of the result).
+// 1/c for a positive count: hardware reciprocal plus one Newton step (2e-15 off
+// at most, far below the float32 rounding of the result).
 __device__ __forceinline__ double recip(int c) {
   const double dc = (double)c;
   double r = __builtin_amdgcn_rcp(dc);
@@ -311,8 +311,8 @@ __device__ __forceinline__ double sqrt_for_f32(double v) {
 }
 
 // float32 moment outputs are formed in float64 with 1/c and 1/(c - 1) from
-// refined reciprocals (about 1 ULP of float64 each, far below the float32
-// rounding of the result) and masked by a select, so they compile without a
+// refined reciprocals (2e-15 off at most, far below the float32 rounding of
+// the result) and masked by a select, so they compile without a
 // branch or a float64 division; float64 outputs keep the reference's divisions.
 template <typename T, int KIND>
 struct VarTraits {
