@@ -280,9 +280,9 @@ __global__ __launch_bounds__(kWave) void move_cols_kernel(MoveColsArgs A) {
 // Positions per wave, or 0 where the general path is the better one: fewer
 // than half a wave of columns, or a window that would be summed anew (and its
 // tails read) for too few positions. A grid of about 8192 waves where the array
-// holds that many of at least 64 positions (LDS lets a CU hold 9 of them at a
-// time where whole lines are written, else 19: about half of the grid, so that
-// the rest evens out the end); at most 4096 positions (2048 for float64), after
+// holds that many of at least 64 positions (a CU holds 9 of them at a time where
+// whole lines are written, by LDS, else 8 to 19, by registers and LDS: the rest
+// of the grid evens out the end); at most 4096 positions (2048 for float64), after
 // which the running sums start afresh, as the tiles of moving.hip do.
 int64_t move_cols_chunk(int elem, int64_t outer, int64_t n, int64_t cols, int64_t window) {
   if (outer <= 0 || n <= 0 || cols < 32 || window <= 0) return 0;

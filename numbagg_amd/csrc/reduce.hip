@@ -607,11 +607,11 @@ struct ColShape {
 };
 
 // Vectors of 16 bytes where they fill at least half a wave; columns split
-// evenly over the tiles. Row splits: a grid of about 2048 workgroups, 8 per CU
-// (4-byte types in vectors keep 32 KiB of partials in LDS, so 5 of them are
-// resident at a time; 8-byte types and single columns all 8), each split at
-// least two unrolled steps of every row lane. (3653, 65160) float32 nanvar takes
-// 255 tiles by 8 splits.
+// evenly over the tiles. Row splits: a grid of about 2048 workgroups, 8 per CU,
+// of which the registers (and the 32 KiB of LDS of 4-byte vectors) let 4 to 5 be
+// resident with vectors, 7 to 8 with single columns; each split at least two
+// unrolled steps of every row lane. (3653, 65160) float32 nanvar takes 255 tiles
+// by 8 splits.
 inline ColShape col_shape(int64_t outer, int64_t n, int64_t cols, int elem) {
   ColShape c{};
   const int vmax = 16 / elem;
