@@ -376,3 +376,23 @@ def test_exp_var_is_as_accurate_as_cov(gpu_lib, dtype):
     rms = [np.sqrt(np.mean(((got - want)[at] / unit[at]) ** 2))
            for got in (nb.move_exp_nanvar(x, alpha=0.01), nb.move_exp_nancov(x, x, alpha=0.01))]
     assert rms[0] <= 1.1 * rms[1], rms
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("rows", [127, 128, 129, 135])
+def test_exp_row_slots(gpu_lib, monkeypatch, rows, dtype):
+    """One pass over a number of rows that its grid rounds up to a multiple of
+    8 (from 128 on): what two passes give, with this file's bars."""
+    import numbagg_amd as nb
+
+    x = walk_array(rows, 20_001, seed=rows, dtype=dtype, offset=5.0)
+    y = walk_array(rows, 20_001, seed=rows + 1, dtype=dtype, offset=-3.0)
+    scale = float(np.nanmax(np.abs(x)))
+    for func in FUNCS1 + FUNCS2:
+        out = {}
+        for two in ("0", "1"):
+            monkeypatch.setenv("NBG_EXP_TWO_PASS", two)
+            out[two] = getattr(nb, func)(*_args(func, x, y), alpha=0.05)
+        bar = 2e-9 if func in MOMENTS else 2e-12
+        assert np.array_equal(np.isnan(out["0"]), np.isnan(out["1"])), func
+        assert_allclose(out["0"], out["1"], rtol=bar, atol=bar * (scale**2 if func in MOMENTS else scale), err_msg=func)
